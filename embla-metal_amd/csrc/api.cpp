@@ -246,7 +246,7 @@ int embla_decode_int8_qraw(const void* qraw, const void* g1, const void* g2, int
         if (!ws || ws_bytes < embla_workspace_bytes(max_s, n_q)) return EMBLA_ERR_WORKSPACE;
         if ((size_t)C * n_q * kPartStride * 4 > part_bytes(max_s, n_q)) return EMBLA_ERR_WORKSPACE;
     }
-    Workspace w = ws ? carve(ws, max_s, n_q) : Workspace{nullptr, nullptr, nullptr};
+    Workspace w = ws ? carve(ws, max_s, n_q) : Workspace{nullptr, nullptr};
     FullDecodeArgs a;
     a.q = (const uint16_t*)qraw;
     a.g1 = (const uint16_t*)g1;
