@@ -47,7 +47,10 @@ def _compile(src: Path) -> Path:
 
 
 def build(verbose: bool = False) -> Path:
-    """Compiles every source and links the shared library; returns its path."""
+    """Compiles every source and links the shared library; returns its path. The built libraries go
+    first: after a failed build nothing loads, instead of an older library than the sources."""
+    for lib in (LIB, HOST_LIB, PROBE_LIB):
+        lib.unlink(missing_ok=True)
     OBJ.mkdir(exist_ok=True)
     srcs = sources()
     with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:

@@ -13,6 +13,7 @@ BIN = HERE / "test_attention_engine"
 
 
 def build() -> Path:
+    BIN.unlink(missing_ok=True)   # a failed build leaves no older binary to be run
     obj = HERE / "_build"
     obj.mkdir(exist_ok=True)
     orc_o = obj / "oracle.o"
