@@ -16,8 +16,14 @@
 //      -128·2^-24·Σq (a constant of the row, as three fp16 parts), so a chain ends at 2^-24 q·k.
 //   A step is KB blocks: with one row block, two blocks' independent score chains.
 //   weights: with u = relu(2^-24 q·k)², a key's K scale enters as a = (2^24 scale/√128)², its V scale
-//      with it as a·vscale: Σ += u a and P = u a vscale, in fp32; V itself is widened exactly
-//      (biased V sums would cancel over a long context).
+//      with it as a·vscale: Σ += u a in fp32, and P = u a vscale enters the product as fp16; V itself
+//      is widened exactly (biased V sums would cancel over a long context).
+//   P's range: a weight is as small as its score and V's scale make it, and the sink keeps small ones
+//      from being normalised away, so powers of two bring P into fp16's normal range whatever they
+//      are: 2^n a query row, which puts its largest |q| in [2^12, 2^13) (then u <= 8²; the sink is
+//      scaled with it), and 2^-e a wave, which keeps a·vscale <= 2^9 for the keys it has seen (raised
+//      in steps when a key exceeds it, O with it; two instructions a block when none does). Without
+//      them scores a tenth of unit size over V of 0.001 lost 3% of the result, over 0.0001 half.
 #include "common.hpp"
 #include "embla_internal.hpp"
 
@@ -46,12 +52,19 @@ __device__ __forceinline__ float xchg_xor32(float v) {
     return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
 }
 
+/// The larger of each half, unsigned.
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
+    typedef uint16_t us2_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2_t, a), __builtin_bit_cast(us2_t, b)));
+}
+
 template <int RB, int KB>
 __global__ __launch_bounds__(64 * R2_WAVES, 1) void relu2_prefill_kernel(PrefillArgs a) {
     __shared__ __attribute__((aligned(16))) float red[R2_WAVES / 2][32][R2_ROW];
     __shared__ __attribute__((aligned(16))) h8_t qs[RB][9][64];
     __shared__ __attribute__((aligned(16))) float scl[R2_WAVES][KB][64];
     __shared__ float lred[R2_WAVES][32 * RB];
+    __shared__ float sink[32 * RB];           // √128 in the row's scale
     constexpr int TOK = R2_TOK * RB;
     // consecutive workgroups: one kv head an XCD (n_kv divides the XCD count), the longest rows first
     const int kvh = blockIdx.x % a.n_kv, tb = gridDim.x / a.n_kv - 1 - blockIdx.x / a.n_kv;
@@ -102,13 +115,32 @@ __global__ __launch_bounds__(64 * R2_WAVES, 1) void relu2_prefill_kernel(Prefill
     if (w < RB) {
         const int tok = min(t0 + R2_TOK * w + (r >> 3), a.T - 1), hq = kvh * R2_GQ + (r & 7);
         const uint16_t* qr = a.q + (size_t)tok * a.q_tok_stride + (size_t)hq * a.q_head_stride;
-        float sum = 0.0f;
+        u4_t raw[8];
+        uint32_t mag = 0;   // the largest magnitude, as bf16 bits (past 0x7F80: a NaN)
 #pragma unroll
         for (int s = 0; s < 8; s++) {
-            const h8_t x = bf8_to_h8(ld16(qr + 32 * (s >> 1) + 16 * h + 8 * (s & 1)));
-            qs[w][s][lane] = x;
+            raw[s] = ld16(qr + 32 * (s >> 1) + 16 * h + 8 * (s & 1));
 #pragma unroll
-            for (int e = 0; e < 8; e++) sum += (float)x[e];
+            for (int i = 0; i < 4; i++) mag = pk_max_u16(mag, raw[s][i] & 0x7FFF7FFFu);
+        }
+        mag = max(mag & 0xFFFFu, mag >> 16);
+        mag = max(mag, __float_as_uint(xchg_xor32(__uint_as_float(mag))));
+        const int n = min(max(12 - ((int)(mag >> 7) - 127), -60), 60);
+        const float up = __uint_as_float((uint32_t)(127 + n) << 23);   // 2^n
+        // a row with an infinity (or past the range of n) has no finite output, one with a NaN no weight
+        if (h == 0)
+            sink[32 * w + r] = bf2f((uint16_t)mag) * up >= 65504.0f ? __uint_as_float(0x7FC00000u) : 11.313708498984761f * up * up;
+        float sum = 0.0f;
+        const h2_t ones = {(_Float16)1.0f, (_Float16)1.0f};
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            h2_t x[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                x[i] = (h2_t){(_Float16)(__uint_as_float(raw[s][i] << 16) * up), (_Float16)(__uint_as_float(raw[s][i] & 0xFFFF0000u) * up)};
+                sum = __builtin_amdgcn_fdot2(x[i], ones, sum, false);
+            }
+            qs[w][s][lane] = *(const h8_t*)x;
         }
         // the bias step: -128·2^-24·Σq against A's 2^-12, as the sum of three fp16 parts
         const float v = sum_xor32(sum) * (-128.0f * 0x1p-12f);
@@ -121,6 +153,7 @@ __global__ __launch_bounds__(64 * R2_WAVES, 1) void relu2_prefill_kernel(Prefill
     const h8_t aone = {one, one, one, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
     f16_t O[RB][4];
     float lsum[RB];
+    float lim = 0.0f, esc = 1.0f;   // uniform: the a·vscale that 2^-e allows for, and 2^-e
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
         lsum[rb] = 0.0f;
@@ -136,14 +169,16 @@ __global__ __launch_bounds__(64 * R2_WAVES, 1) void relu2_prefill_kernel(Prefill
         // which made the wait for K one for V too)
         load_v(k);
         __builtin_amdgcn_sched_barrier(0);
+        float kv[KB];
 #pragma unroll
         for (int i = 0; i < KB; i++) {
             // lane l < 32: key l's a = (2^24 scale / √128)²; lane 32 + l: a times its V scale; both 0
-            // past the workgroup's last key, whose scales may never have been written
-            const float sc = k0 + 32 * i + r <= last ? scv[i] : 0.0f;
+            // outside the workgroup's keys, whose scales may never have been written
+            const float sc = (uint32_t)(k0 + 32 * i - lo_wg + r) <= (uint32_t)(last - lo_wg) ? scv[i] : 0.0f;
             const float ks = sc * (0.08838834764831845f * 0x1p24f), k2 = ks * ks;
             const float o = xchg_xor32(k2);
-            scl[w][i][lane] = h ? o * sc : k2;
+            kv[i] = o * sc;   // (of use where h = 1)
+            scl[w][i][lane] = h ? kv[i] * esc : k2;
         }
         f16_t s[KB][RB];
 #pragma unroll
@@ -163,6 +198,23 @@ __global__ __launch_bounds__(64 * R2_WAVES, 1) void relu2_prefill_kernel(Prefill
         __builtin_amdgcn_sched_barrier(0);
         load_k(k + R2_WAVES);
         __builtin_amdgcn_sched_barrier(0);
+        float top = fabsf(kv[0]);
+#pragma unroll
+        for (int i = 1; i < KB; i++) top = fmaxf(top, fabsf(kv[i]));
+        if (__ballot(top > lim) >> 32) {   // a key past what 2^-e allows for: e rises, O and the scales with it
+            top = wave_bfly(h ? top : 0.0f, [](float x, float y) { return fmaxf(x, y); });
+            const int ex = min(max((int)(__float_as_uint(top) >> 23) - 127, -100), 100) + 1;
+            const float to = __uint_as_float((uint32_t)(127 + 9 - ex) << 23), f = to / esc;
+            lim = __uint_as_float((uint32_t)(127 + ex) << 23);
+            esc = to;
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) O[rb][i] *= f;
+            if (h)
+#pragma unroll
+                for (int i = 0; i < KB; i++) scl[w][i][lane] = kv[i] * esc;
+        }
         wave_lds_sync();
         // item e = 4c + j of block i is key k0 + 32i + 8c + 4h + j
         if (k0 + 32 * KB - 1 > a.p0 + t0 || k0 < lo_all) {   // uniform: not every row sees every key
@@ -186,14 +238,14 @@ __global__ __launch_bounds__(64 * R2_WAVES, 1) void relu2_prefill_kernel(Prefill
             h8_t pb[RB][2];
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                const f4_t ka = *(const f4_t*)&scl[w][i][8 * c + 4 * h], kv = *(const f4_t*)&scl[w][i][32 + 8 * c + 4 * h];
+                const f4_t ka = *(const f4_t*)&scl[w][i][8 * c + 4 * h], kp = *(const f4_t*)&scl[w][i][32 + 8 * c + 4 * h];
 #pragma unroll
                 for (int rb = 0; rb < RB; rb++)
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
                         const float t = fmaxf(s[i][rb][4 * c + j], 0.0f), u = t * t;
                         lsum[rb] = __builtin_fmaf(u, ka[j], lsum[rb]);
-                        pb[rb][c & 1][4 * (c >> 1) + j] = (_Float16)(u * kv[j]);
+                        pb[rb][c & 1][4 * (c >> 1) + j] = (_Float16)(u * kp[j]);
                     }
             }
 #pragma unroll
@@ -210,7 +262,7 @@ __global__ __launch_bounds__(64 * R2_WAVES, 1) void relu2_prefill_kernel(Prefill
         wave_lds_sync();   // the scales are read before the next step's replace them
     }
 
-    // ---- the waves' sums: waves 4 .. 7 hand theirs to waves 0 .. 3, whose four are then added in the
+    // ---- the waves' sums, each times its 2^e: waves 4 .. 7 hand theirs to waves 0 .. 3, whose four are then added in the
     // output pass, a row block at a time. O^T row block i, item (b, e): row r' = 8b + 4h + e is dim
     // 8 (r' % 16) + 4 (i / 2) + 2 (r' / 16) + i % 2, so the lane holds the 8 dims of n = r' % 16 whole
 #pragma unroll
@@ -218,6 +270,7 @@ __global__ __launch_bounds__(64 * R2_WAVES, 1) void relu2_prefill_kernel(Prefill
         const float l = sum_xor32(lsum[rb]);
         if (h == 0) lred[w][32 * rb + r] = l;
     }
+    const float back = 1.0f / esc;
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
         auto slot = [&](int b, int e, int half) -> f4_t* {
@@ -225,7 +278,7 @@ __global__ __launch_bounds__(64 * R2_WAVES, 1) void relu2_prefill_kernel(Prefill
         };
         auto part = [&](int b, int e, int half) -> f4_t {
             const f16_t *x = &O[rb][2 * half], *y = &O[rb][2 * half + 1];
-            return (f4_t){(*x)[4 * b + e], (*y)[4 * b + e], (*x)[8 + 4 * b + e], (*y)[8 + 4 * b + e]};
+            return (f4_t){(*x)[4 * b + e], (*y)[4 * b + e], (*x)[8 + 4 * b + e], (*y)[8 + 4 * b + e]} * back;
         };
         if (rb > 0) __syncthreads();   // the previous row block's output pass has read the slots
         if (w >= R2_WAVES / 2) {
@@ -243,7 +296,7 @@ __global__ __launch_bounds__(64 * R2_WAVES, 1) void relu2_prefill_kernel(Prefill
         __syncthreads();
         const int rr = tid >> 4, d0 = 8 * (tid & 15), ot = t0 + R2_TOK * rb + (rr >> 3);   // 8 dims a thread
         if (ot < a.T) {
-            float den = 11.313708498984761f;
+            float den = sink[32 * rb + rr];
 #pragma unroll
             for (int i = 0; i < R2_WAVES; i++) den += lred[i][32 * rb + rr];
             const float inv = 1.0f / den;
