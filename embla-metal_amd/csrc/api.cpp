@@ -35,8 +35,8 @@ int env_int(const char* name, int dflt) {
     return atoi(s);
 }
 
-/// Bytes of one key-range split's partial records of T tokens and n_q heads (prefill.hip's PPH).
-size_t split_bytes(int T, int n_q) { return (size_t)T * n_q * 68 * 4; }
+/// Bytes of one key-range split's partial records of T tokens and n_q heads (prefill.hip's PPF, PPH).
+size_t split_bytes(int T, int n_q, bool rec32 = true) { return (size_t)T * n_q * (rec32 ? 132 : 68) * 4; }
 
 /// Key-range splits a prefill workspace of T tokens and n_q heads has room for: as many as give every
 /// CU a workgroup (at least 64 tokens of 4 heads each), at most kPrefillMaxSplits.
@@ -52,8 +52,10 @@ int splits_room(int T, int n_q) {
 /// one workgroup's pace (4 us a 128-key tile): with two splits at most, 193 tokens after 7003 keys took
 /// 103 us and 40 after 30000 373; 35.7 and 33 with this. Two tiles a split at least: 35.8 and 33, but
 /// 33.1 against 31.4 for 400 tokens after 1000 keys and 21.5 against 18.9 for 60 over a window of 512.
+/// Two splits of 512 keys or more keep fp16 records, all others fp32 ones (rec32).
 /// EMBLA_PREFILL_SPLITS caps it (tuning).
-int prefill_splits(const void* ws, size_t ws_bytes, int T, int n_q, int blocks, int tiles) {
+int prefill_splits(const void* ws, size_t ws_bytes, int T, int n_q, int blocks, int tiles, bool& rec32) {
+    rec32 = false;
     if (!ws || ws_bytes < (size_t)kPrefillSplits * T * n_q * kPartStride * 4) return 1;
     static const int cap = env_int("EMBLA_PREFILL_SPLITS", kPrefillMaxSplits);
     const size_t own = embla_prefill_workspace_bytes(T, n_q);   // (a staged copy follows the partials)
@@ -62,6 +64,7 @@ int prefill_splits(const void* ws, size_t ws_bytes, int T, int n_q, int blocks, 
     if (ns > cap) ns = cap;
     if (ns > kPrefillMaxSplits) ns = kPrefillMaxSplits;
     if (ns > (int)room) ns = (int)room;
+    rec32 = ns > 2 || tiles < 8;
     return ns < 1 ? 1 : ns;
 }
 
@@ -653,7 +656,7 @@ int embla_prefill_int8(const void* q, int q_dtype, long q_tok_stride, long q_hea
     const int gqw = n_q / n_kv, rows_wg = gqw >= 1 && gqw <= 8 ? 32 * (8 / gqw) : 32;   // query rows a workgroup
     const int blocks = (T + rows_wg - 1) / rows_wg * n_kv;
     a.nsplit = prefill_splits(ws, ws_bytes, T, n_q, blocks,
-                              window > 0 ? min((p0 + T) / 64, (window + 63) / 64 + 1) : (p0 + T) / 64);
+                              window > 0 ? min((p0 + T) / 64, (window + 63) / 64 + 1) : (p0 + T) / 64, a.rec32);
     a.part = (float*)ws;
     a.kring = nullptr; a.vring = nullptr; a.R = 0; a.qg = nullptr;
     a.relu2 = weights == EMBLA_RELU2_SINK; a.scale32 = scale_dtype == EMBLA_F32;
@@ -719,7 +722,7 @@ int embla_prefill_ring(const void* q, int dtype, long q_tok_stride, long q_head_
     a.T = T; a.p0 = p0; a.max_s = ring; a.n_q = n_q; a.n_kv = n_kv; a.window = window;
     const int gqw = n_q / n_kv, rows_wg = gqw >= 1 && gqw <= 8 ? 32 * (8 / gqw) : 32;   // query rows a workgroup
     const int blocks = (T + rows_wg - 1) / rows_wg * n_kv;
-    a.nsplit = prefill_splits(ws, ws_bytes, T, n_q, blocks, (window + 63) / 64 + 1);
+    a.nsplit = prefill_splits(ws, ws_bytes, T, n_q, blocks, (window + 63) / 64 + 1, a.rec32);
     a.part = (float*)ws;
     a.relu2 = false; a.scale32 = false; a.q_bf16 = dtype == EMBLA_BF16; a.out_bf16 = dtype == EMBLA_BF16;
     a.kring = (const uint16_t*)kring; a.vring = (const uint16_t*)vring; a.R = ring; a.qg = (const uint16_t*)qg;

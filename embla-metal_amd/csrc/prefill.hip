@@ -52,13 +52,16 @@ struct __attribute__((aligned(16))) PrefillSmem {
     _Float16 vt[2][NSUB * VTILE];
 };
 
-// a split's partial record (floats): O / l as 128 fp16, then m and l in fp32, padded to 16 bytes:
-// half the bytes of an fp32 O for the split pass to write and the merge to read. O / l is a convex
-// combination of V rows (l is the split's own weight sum), and
+// a split's partial record (floats): O, m and l in fp32, padded to 16 bytes (PPF), or O / l as 128
+// fp16, then m and l (PPH): half the bytes for the split pass to write and the merge to read, taken
+// where a long chunk's range splits in two (its records are 17 MB at 2048 tokens of 16 heads). O / l
+// is a convex combination of V rows (l is the split's own weight sum), and
 // every instance's P·V product already takes V as fp16: int8 V exactly, 16-bit ring V as a copy
 // (fp16 rings) or widened to fp16 in staging (bf16 rings, bf8_to_h8: exact for |v| in
-// [2^-14, 65504]). So the fp16 record loses no range that the product keeps.
-constexpr int PPH = 68;
+// [2^-14, 65504]). So the fp16 record loses no range that the product keeps, only a rounding to 11
+// bits that bf16 outputs do not show and fp16 ones do (60 tokens after 5000 keys in 39 splits, error
+// against 64 bits: 5.54e-4 with fp16 records, 5.15e-4 with fp32 ones, 5.14e-4 unsplit).
+constexpr int PPH = 68, PPF = HD + 4;
 #ifndef PF_PRIO
 // wave priority raised over the score chains (1), the P·V products (2): with two waves a SIMD
 // entering each tile together, the raised one issues its chain first and the two drift into
@@ -544,7 +547,30 @@ __global__ __launch_bounds__(64 * PF_WAVES, 1) void prefill_int8_kernel(PrefillA
     const bool coalesced = ((uintptr_t)a.o % 16) == 0 && a.o_tok_stride % 8 == 0 && a.o_head_stride % 8 == 0;
     __syncthreads();
     float* stg = (float*)&sm;
-    if (a.nsplit > 1) {   // this split's partial records: O / l (fp16), m, l
+    auto records = [&](auto len) {   // the staged records of len floats to this split's rows
+        constexpr int PP = decltype(len)::value, TS = GQ * PP + 4;
+        constexpr int CPT = GQ * PP / 4;   // 16-byte chunks a token
+        float* pz = a.part + ((size_t)z * a.T + wt0) * a.n_q * PP + (size_t)kvh * GQ * PP;
+        __syncthreads();
+        for (int cidx = tid; cidx < ntok * CPT; cidx += NT) {
+            const int t = cidx / CPT, off = 4 * (cidx % CPT);
+            *(f4_t*)(pz + (size_t)t * a.n_q * PP + off) = *(const f4_t*)(stg + t * TS + off);
+        }
+    };
+    if (a.nsplit > 1 && a.rec32) {   // this split's partial records: O, m, l
+        constexpr int TS = GQ * PPF + 4;   // floats a token: the 16-byte writes of 16 rows on distinct banks
+        static_assert(32 * RB * TS * 4 <= sizeof(PrefillSmem), "the workgroup's records fit the tile buffers");
+        float* rec = stg + tl * TS + hl * PPF;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int bb = 0; bb < 4; bb++)
+                *(f4_t*)(rec + 32 * i + 8 * bb + 4 * h) = (f4_t){O[i][4 * bb], O[i][4 * bb + 1], O[i][4 * bb + 2], O[i][4 * bb + 3]};
+        if (h == 0) *(f4_t*)(rec + HD) = (f4_t){m, lsum, 0.0f, 0.0f};
+        records(std::integral_constant<int, PPF>{});
+        return;
+    }
+    if (a.nsplit > 1) {   // O / l (fp16), m, l
         constexpr int TS = GQ * PPH + 4;   // floats a token: the 8-byte writes of 16 rows on distinct banks
         float* rec = stg + tl * TS + hl * PPH;
         const float il = lsum > 0.0f ? 1.0f / lsum : 0.0f;
@@ -559,13 +585,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 1) void prefill_int8_kernel(PrefillA
                 *(u2_t*)(r16 + 32 * i + 8 * bb + 4 * h) = pk;
             }
         if (h == 0) *(f4_t*)(rec + HD / 2) = (f4_t){m, lsum, 0.0f, 0.0f};
-        __syncthreads();
-        constexpr int CPT = GQ * PPH / 4;   // 16-byte chunks a token
-        float* pz = a.part + ((size_t)z * a.T + wt0) * a.n_q * PPH + (size_t)kvh * GQ * PPH;
-        for (int cidx = tid; cidx < ntok * CPT; cidx += NT) {
-            const int t = cidx / CPT, off = 4 * (cidx % CPT);
-            *(f4_t*)(pz + (size_t)t * a.n_q * PPH + off) = *(const f4_t*)(stg + t * TS + off);
-        }
+        records(std::integral_constant<int, PPH>{});
         return;
     }
     if (!coalesced) {   // (uniform) strides that a 16-byte store cannot take: one row a lane
@@ -604,37 +624,80 @@ __global__ __launch_bounds__(64 * PF_WAVES, 1) void prefill_int8_kernel(PrefillA
     }
 }
 
-/// Merges the nsplit partial records of (token, head): 32 lanes a row, 4 dims a lane (8-byte loads),
-/// 8 rows a workgroup: rows (blockIdx.x * 8 + tid / 32) of head blockIdx.y.
-template <bool OBF>
+/// Merges the nsplit <= 4 G partial records of (token, head): 16 lanes of 8 dims times G groups of
+/// records a row (a lane takes up to 4 records; one summing 64 would be a serial chain). G = 1: 16 rows
+/// a workgroup. G = 4: a wave a row, its 16-lane rows the groups. G = 16: a workgroup a row, the four
+/// waves' shares meeting in LDS.
+template <bool OBF, bool F32, int G>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
-    // 16 lanes a (token, head): 8 dims a lane, one 16-byte load of a split's O / l record
-    const int lane = threadIdx.x & 15, tok = blockIdx.x * 16 + (threadIdx.x >> 4), hq = blockIdx.y;
+    constexpr int PP = F32 ? PPF : PPH;
+    const int lane = threadIdx.x & 15, slot = threadIdx.x >> 4, grp = slot % G, hq = blockIdx.y;
+    const int tok = blockIdx.x * (16 / G) + slot / G;
     if (tok >= a.T) return;
-    float M = NEG_INF, mz[4], lz[4];
-    u4_t v[4];
+    float M = NEG_INF, mz[4], lz[4], v[4][8];
 #pragma unroll
-    for (int z = 0; z < 4; z++) {
+    for (int i = 0; i < 4; i++) {
+        const int z = grp + G * i;
+        mz[i] = NEG_INF;
         if (z < a.nsplit) {
-            const float* pp = a.part + (((size_t)z * a.T + tok) * a.n_q + hq) * PPH;
-            v[z] = ld16((const uint16_t*)pp + 8 * lane);   // O / l, fp16
-            const u2_t ml = ld8(pp + HD / 2);
-            mz[z] = __uint_as_float(ml[0]);
-            lz[z] = __uint_as_float(ml[1]);
-            M = fmaxf(M, mz[z]);
+            const float* pp = a.part + (((size_t)z * a.T + tok) * a.n_q + hq) * PP;
+            const u2_t ml = ld8(pp + (F32 ? HD : HD / 2));
+            mz[i] = __uint_as_float(ml[0]);
+            lz[i] = __uint_as_float(ml[1]);
+            if constexpr (F32) {
+                const u4_t x = ld16(pp + 8 * lane), y = ld16(pp + 8 * lane + 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    v[i][e] = __uint_as_float(x[e]);
+                    v[i][4 + e] = __uint_as_float(y[e]);
+                }
+            } else {
+                const u4_t x = ld16((const uint16_t*)pp + 8 * lane);
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[i][e] = h2f((uint16_t)(x[e / 2] >> (16 * (e & 1))));
+            }
+            M = fmaxf(M, mz[i]);
         }
+    }
+    __shared__ __attribute__((aligned(16))) float acc4[G == 16 ? 4 : 1][HD];
+    __shared__ float m4[4], l4[4];
+    const int w = threadIdx.x >> 6;
+    if constexpr (G > 1) M = max_rows(M);
+    if constexpr (G == 16) {
+        if ((threadIdx.x & 63) == 0) m4[w] = M;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; i++) M = fmaxf(M, m4[i]);
     }
     float L = 0.0f, acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int z = 0; z < 4; z++) {
-        if (z < a.nsplit) {
-            // split z's share: its l, rescaled to the common maximum
-            const float f = lz[z] * (mz[z] == NEG_INF ? 0.0f : exp2f(mz[z] - M));
-            L += f;
+    for (int i = 0; i < 4; i++) {
+        if (grp + G * i < a.nsplit && mz[i] != NEG_INF) {
+            // the split's share, rescaled to the common maximum: its l, and its O or (O / l) l
+            const float f = exp2f(mz[i] - M), fo = F32 ? f : lz[i] * f;
+            L += lz[i] * f;
 #pragma unroll
-            for (int i = 0; i < 8; i++) acc[i] += h2f((uint16_t)(v[z][i / 2] >> (16 * (i & 1)))) * f;
+            for (int e = 0; e < 8; e++) acc[e] += v[i][e] * fo;
         }
     }
+    if constexpr (G > 1) {
+        L = sum_rows(L);
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] = sum_rows(acc[e]);
+    }
+    if constexpr (G == 16) {
+        if ((threadIdx.x & 63) < 16) {
+            *(f4_t*)&acc4[w][8 * lane] = (f4_t){acc[0], acc[1], acc[2], acc[3]};
+            *(f4_t*)&acc4[w][8 * lane + 4] = (f4_t){acc[4], acc[5], acc[6], acc[7]};
+            if (lane == 0) l4[w] = L;
+        }
+        __syncthreads();
+        L = (l4[0] + l4[1]) + (l4[2] + l4[3]);
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            acc[e] = (acc4[0][8 * lane + e] + acc4[1][8 * lane + e]) + (acc4[2][8 * lane + e] + acc4[3][8 * lane + e]);
+    }
+    if (grp != 0) return;
     const float inv = 1.0f / L;
     uint16_t* orow = a.o + (size_t)tok * a.o_tok_stride + (size_t)hq * a.o_head_stride;
     u4_t pk;
@@ -643,59 +706,10 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
         pk[i] = (uint32_t)f2a<OBF>(acc[2 * i] * inv) | ((uint32_t)f2a<OBF>(acc[2 * i + 1] * inv) << 16);
     if (((uintptr_t)orow & 15) == 0) {
         *(u4_t*)(orow + 8 * lane) = pk;
-    } else {   // a token or head stride that breaks 16-byte alignment (4-byte aligned always)
+    } else {   // a token or head stride that breaks 16-byte alignment
         *(u2_t*)(orow + 8 * lane) = (u2_t){pk[0], pk[1]};
         *(u2_t*)(orow + 8 * lane + 4) = (u2_t){pk[2], pk[3]};
     }
-}
-
-/// The same merge of 5 to 64 records: a workgroup a (token, head), 16 lanes of 8 dims by 16 groups of
-/// records, whose sums meet in LDS (a thread summing 64 records would be one serial chain).
-template <bool OBF>
-__global__ __launch_bounds__(256) void prefill_merge_wide_kernel(PrefillArgs a) {
-    const int lane = threadIdx.x & 15, grp = threadIdx.x >> 4, tok = blockIdx.x, hq = blockIdx.y;
-    __shared__ __attribute__((aligned(16))) float acc[16][HD + 4];
-    __shared__ float gm[16], gl[16];
-    float mz[4], lz[4], M = NEG_INF;
-    u4_t v[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int z = grp + 16 * i;
-        mz[i] = NEG_INF;
-        if (z < a.nsplit) {
-            const float* pp = a.part + (((size_t)z * a.T + tok) * a.n_q + hq) * PPH;
-            v[i] = ld16((const uint16_t*)pp + 8 * lane);
-            const u2_t ml = ld8(pp + HD / 2);
-            mz[i] = __uint_as_float(ml[0]);
-            lz[i] = __uint_as_float(ml[1]);
-            M = fmaxf(M, mz[i]);
-        }
-    }
-    float L = 0.0f, s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if (grp + 16 * i < a.nsplit && mz[i] != NEG_INF) {
-            const float f = lz[i] * exp2f(mz[i] - M);
-            L += f;
-#pragma unroll
-            for (int e = 0; e < 8; e++) s[e] += h2f((uint16_t)(v[i][e / 2] >> (16 * (e & 1)))) * f;
-        }
-    }
-    *(f4_t*)&acc[grp][8 * lane] = (f4_t){s[0], s[1], s[2], s[3]};
-    *(f4_t*)&acc[grp][8 * lane + 4] = (f4_t){s[4], s[5], s[6], s[7]};
-    if (lane == 0) { gm[grp] = M; gl[grp] = L; }
-    __syncthreads();
-    if (threadIdx.x >= HD) return;
-    float top = NEG_INF, sum = 0.0f, l = 0.0f;
-#pragma unroll
-    for (int g = 0; g < 16; g++) top = fmaxf(top, gm[g]);
-#pragma unroll
-    for (int g = 0; g < 16; g++) {
-        const float f = gm[g] == NEG_INF ? 0.0f : exp2f(gm[g] - top);
-        l += gl[g] * f;
-        sum += acc[g][threadIdx.x] * f;
-    }
-    a.o[(size_t)tok * a.o_tok_stride + (size_t)hq * a.o_head_stride + threadIdx.x] = f2a<OBF>(sum / l);
 }
 
 int launch_prefill_int8(const PrefillArgs& a, hipStream_t st) {
@@ -790,16 +804,17 @@ int launch_prefill_prestaged(const PrefillArgs& a0, uint16_t* k16, uint16_t* v16
     return launch_prefill_tail(a, st);
 }
 
+template <bool OBF>
+static void launch_prefill_merge(const PrefillArgs& a, hipStream_t st) {
+    auto grid = [&](int rows) { return dim3((a.T + rows - 1) / rows, a.n_q); };
+    if (!a.rec32) hipLaunchKernelGGL((prefill_merge_kernel<OBF, false, 1>), grid(16), dim3(256), 0, st, a);
+    else if (a.nsplit <= 4) hipLaunchKernelGGL((prefill_merge_kernel<OBF, true, 1>), grid(16), dim3(256), 0, st, a);
+    else if (a.nsplit <= 16) hipLaunchKernelGGL((prefill_merge_kernel<OBF, true, 4>), grid(4), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((prefill_merge_kernel<OBF, true, 16>), grid(1), dim3(256), 0, st, a);
+}
+
 int launch_prefill_tail(const PrefillArgs& a, hipStream_t st) {
-    if (a.nsplit > 4) {
-        const dim3 mg(a.T, a.n_q);
-        if (a.out_bf16) hipLaunchKernelGGL(prefill_merge_wide_kernel<true>, mg, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL(prefill_merge_wide_kernel<false>, mg, dim3(256), 0, st, a);
-    } else if (a.nsplit > 1) {
-        const dim3 mg((a.T + 15) / 16, a.n_q);
-        if (a.out_bf16) hipLaunchKernelGGL(prefill_merge_kernel<true>, mg, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL(prefill_merge_kernel<false>, mg, dim3(256), 0, st, a);
-    }
+    if (a.nsplit > 1) a.out_bf16 ? launch_prefill_merge<true>(a, st) : launch_prefill_merge<false>(a, st);
     return hipGetLastError() == hipSuccess ? EMBLA_OK : EMBLA_ERR_HIP;
 }
 

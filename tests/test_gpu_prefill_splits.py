@@ -23,13 +23,13 @@ def torch_gpu():
 # 64-key tiles (p0 + T) / 64, halved: the splits of a chunk of few workgroups
 @pytest.mark.parametrize("T,p0,window,f16,small_ws,tok_stride", [
     (20, 236, 0, False, False, 2048),      # 2
-    (20, 492, 0, True, False, 2048),       # 4: the last of the narrow merge
-    (20, 620, 0, False, False, 2050),      # 5: the first of the wide one
-    (7, 2042, 0, True, False, 2048),       # 16: one record a lane group
-    (20, 2156, 0, False, False, 2048),     # 17
+    (20, 492, 0, True, False, 2048),       # 4: the last of the merge of a row a lane group
+    (20, 620, 0, False, False, 2050),      # 5: the first of a row a wave
+    (7, 2042, 0, True, False, 2048),       # 16: the last of them
+    (20, 2156, 0, False, False, 2048),     # 17: the first of a row a workgroup
     (1, 8191, 0, False, False, 2048),      # 64, one token
     (65, 5000, 0, False, False, 2049),     # two row blocks: 32 splits
-    (20, 8200, 0, False, True, 2048),      # 64 wanted, room for 7
+    (20, 8200, 0, False, True, 2048),      # 64 wanted, room for 4
     (33, 3000, 700, False, False, 2048),   # a window: 12 tiles, splits that some rows do not see
     (130, 0, 0, True, False, 2048)])       # no prefix
 def test_prefill_splits(torch_gpu, orc, T, p0, window, f16, small_ws, tok_stride):
@@ -56,3 +56,33 @@ def test_prefill_splits(torch_gpu, orc, T, p0, window, f16, small_ws, tok_stride
     ref = orc.prefill_int8(val(q), K, synth.f16_val(ks), V, synth.f16_val(vs), p0, window=window)
     assert_close(got[:, :2048].reshape(T, n_q, 128), ref, what=f"T={T} p0={p0}")
     assert (got[:, 2048:] == 3.0).all()
+
+
+@pytest.mark.parametrize("T,p0", [(193, 130), (60, 440), (193, 800), (60, 5000), (20, 8200)])   # 2, 3, 7, 39, 64 splits at most
+def test_prefill_splits_precision(torch_gpu, T, p0):
+    """A split's sums stay in fp32 on their way to the merge: with fp16 outputs, the error against 64
+    bits is the unsplit call's (1.08 to 1.1 times that with each split's O / l rounded to fp16 too)."""
+    from embla_attn import ops
+    torch = torch_gpu
+    n_q, n_kv, S = 16, 4, p0 + T
+    max_s = (S + 31) // 32 * 32
+    say(f"prefill splits precision T={T} p0={p0}")
+    g = synth.SplitMix64(T + p0)
+    q = synth.f16_bits(g.normal(T * n_q * 128)).reshape(T, n_q, 128)
+    K, V = (g.int8(n_kv * S * 128).reshape(n_kv, S, 128) for _ in range(2))
+    ks, vs = (synth.f16_bits(0.005 + 0.01 * g.uniform(n_kv * S)).reshape(n_kv, S) for _ in range(2))
+    kc, vc = dev(layout.pack_region(K, ks, max_s, "k")), dev(layout.pack_region(V, vs, max_s, "v"))
+    qf = synth.f16_val(q).astype(np.float64)
+    Kf, Vf = (x * synth.f16_val(s).astype(np.float64)[..., None] for x, s in ((K, ks), (V, vs)))
+    ref = np.empty((T, n_q, 128))
+    for h in range(n_q):
+        s = qf[:, h] @ Kf[h // 4].T / np.sqrt(128.0)
+        s[np.arange(S)[None] > p0 + np.arange(T)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        ref[:, h] = p @ Vf[h // 4] / p.sum(1, keepdims=True)
+    err = []
+    for ws in (None, ops.PrefillWorkspace(T, n_q)):
+        o = ops.prefill_int8(dev(q, torch.float16), kc, vc, T, p0, max_s, n_kv, q_dtype=ops.F16, out_dtype=ops.F16, ws=ws)
+        err.append(np.linalg.norm(f16_host(o) - ref) / np.linalg.norm(ref))
+    print(f"[gpu-case] unsplit {err[0]:.3e} split {err[1]:.3e}", flush=True)
+    assert err[1] <= 1.03 * err[0]
