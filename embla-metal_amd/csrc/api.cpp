@@ -35,8 +35,8 @@ int env_int(const char* name, int dflt) {
     return atoi(s);
 }
 
-/// Bytes of one key-range split's partial records of T tokens and n_q heads (prefill.hip's PPF, PPH).
-size_t split_bytes(int T, int n_q, bool rec32 = true) { return (size_t)T * n_q * (rec32 ? 132 : 68) * 4; }
+/// Bytes of one key-range split's partial records of T tokens and n_q heads (prefill.hip's PPF).
+size_t split_bytes(int T, int n_q) { return (size_t)T * n_q * 132 * 4; }
 
 /// Key-range splits a prefill workspace of T tokens and n_q heads has room for: as many as give every
 /// CU a workgroup (at least 64 tokens of 4 heads each), at most kPrefillMaxSplits.
@@ -46,25 +46,41 @@ int splits_room(int T, int n_q) {
     return ns < 1 ? 1 : ns > kPrefillMaxSplits ? kPrefillMaxSplits : ns;
 }
 
-/// Key-range splits of a prefill launch of `blocks` workgroups over `tiles` 64-key tiles: as many as
-/// give every CU one workgroup (8 waves, 2 a SIMD) and every split a 128-key tile, and only with a
-/// workspace for the partial rows. A short chunk's few workgroups otherwise walk the whole key range at
-/// one workgroup's pace (4 us a 128-key tile): with two splits at most, 193 tokens after 7003 keys took
-/// 103 us and 40 after 30000 373; 35.7 and 33 with this. Two tiles a split at least: 35.8 and 33, but
-/// 33.1 against 31.4 for 400 tokens after 1000 keys and 21.5 against 18.9 for 60 over a window of 512.
-/// Two splits of 512 keys or more keep fp16 records, all others fp32 ones (rec32).
-/// EMBLA_PREFILL_SPLITS caps it (tuning).
-int prefill_splits(const void* ws, size_t ws_bytes, int T, int n_q, int blocks, int tiles, bool& rec32) {
+/// Key-range splits of a prefill launch of `blocks` workgroups (at most one a CU at a time), and whether
+/// their records are fp32 (rec32: all but two splits of 512 keys or more, or over a ring whose window
+/// holds as many). A split saves its share of a workgroup's walk, 3.6-4 us a 128-key tile, and costs its
+/// records (written, and read by the merge) and the merge. EMBLA_PREFILL_SPLITS caps it (tuning).
+///  - Two splits where the workgroups leave CUs idle and the range has 512 keys: 700 tokens without a
+///    prefix 27.3 -> 22.6 us. More than half of the CUs' worth (129 on) makes a second round of the
+///    halves, which pays only where the rows' ranges differ much, so that the long ones end late (2112
+///    tokens after 1000 keys 94 -> 86 us, but after 30000 778 -> 864; 3000 over a window of 1024 41 -> 57)
+///    or where the round is nearly full (4000 tokens after 30000 keys 1170 -> 1122).
+///  - More while n² records of the chunk stay under the range's tiles times a constant (a walk of t / n
+///    tiles and n records add up to least there), up to a workgroup a CU and a tile a split, within 6% of
+///    the best count of a sweep of 12 .. 1200 tokens over 0 .. 30000 keys on average 1.8% (at most two
+///    splits: 193 tokens after 7003 keys 103 us, 35.5 with 16; 40 after 30000 373, 31 with 64). Three cost
+///    fp32 records where two have fp16 ones, and only pay where three is what the CUs allow (600 tokens
+///    after 300 keys 25.5 us with 2, 29.2 with 3, 27.4 with 4; 1200 after 3000 73.9 with 2, 61.1 with 3).
+int prefill_splits(const void* ws, size_t ws_bytes, int T, int p0, int window, bool ring, int n_q, int blocks,
+                   bool& rec32) {
     rec32 = false;
     if (!ws || ws_bytes < (size_t)kPrefillSplits * T * n_q * kPartStride * 4) return 1;
+    // the keys of a workgroup's range at most, in 64-key tiles, and of a row on average and at most
+    const long long end = (long long)p0 + T, most = window > 0 ? min(end, (long long)window) : end;
+    const int tiles = (int)(window > 0 ? min(end / 64, (window + 63LL) / 64 + 1) : end / 64);
+    const long long ramp = most - p0 > 0 ? most - p0 : 0;   // rows that see one key more than the last
+    const long long mean = (ramp * (p0 + 1 + most) / 2 + (T - ramp) * most) / T;
     static const int cap = env_int("EMBLA_PREFILL_SPLITS", kPrefillMaxSplits);
+    int ns = 1;
+    if (tiles >= 8 && blocks <= 128) ns = 2;
+    if (tiles >= 8 && blocks > 128 && blocks < 256 && (5 * mean < 4 * most || (window == 0 && blocks > 192))) ns = 2;
+    int more = min(min(256 / blocks, kPrefillMaxSplits), (int)min((long long)(tiles / 2), (mean + 64) / 128));
+    while (more > 1 && (long long)more * more * T * n_q > 16000LL * (tiles / 2)) more--;
+    if (more == 3 && 256 / blocks > 3 && ns == 2) more = 2;
+    ns = max(ns, more);
     const size_t own = embla_prefill_workspace_bytes(T, n_q);   // (a staged copy follows the partials)
-    const size_t room = (ws_bytes < own ? ws_bytes : own) / split_bytes(T, n_q);
-    int ns = 256 / blocks < tiles / 2 ? 256 / blocks : tiles / 2;
-    if (ns > cap) ns = cap;
-    if (ns > kPrefillMaxSplits) ns = kPrefillMaxSplits;
-    if (ns > (int)room) ns = (int)room;
-    rec32 = ns > 2 || tiles < 8;
+    ns = min(min(ns, cap), (int)((ws_bytes < own ? ws_bytes : own) / split_bytes(T, n_q)));
+    rec32 = ns > 2 || (tiles < 8 && !(ring && window >= 448));
     return ns < 1 ? 1 : ns;
 }
 
@@ -655,8 +671,7 @@ int embla_prefill_int8(const void* q, int q_dtype, long q_tok_stride, long q_hea
     // partials cost one merge pass)
     const int gqw = n_q / n_kv, rows_wg = gqw >= 1 && gqw <= 8 ? 32 * (8 / gqw) : 32;   // query rows a workgroup
     const int blocks = (T + rows_wg - 1) / rows_wg * n_kv;
-    a.nsplit = prefill_splits(ws, ws_bytes, T, n_q, blocks,
-                              window > 0 ? min((p0 + T) / 64, (window + 63) / 64 + 1) : (p0 + T) / 64, a.rec32);
+    a.nsplit = prefill_splits(ws, ws_bytes, T, p0, window, false, n_q, blocks, a.rec32);
     a.part = (float*)ws;
     a.kring = nullptr; a.vring = nullptr; a.R = 0; a.qg = nullptr;
     a.relu2 = weights == EMBLA_RELU2_SINK; a.scale32 = scale_dtype == EMBLA_F32;
@@ -722,7 +737,7 @@ int embla_prefill_ring(const void* q, int dtype, long q_tok_stride, long q_head_
     a.T = T; a.p0 = p0; a.max_s = ring; a.n_q = n_q; a.n_kv = n_kv; a.window = window;
     const int gqw = n_q / n_kv, rows_wg = gqw >= 1 && gqw <= 8 ? 32 * (8 / gqw) : 32;   // query rows a workgroup
     const int blocks = (T + rows_wg - 1) / rows_wg * n_kv;
-    a.nsplit = prefill_splits(ws, ws_bytes, T, n_q, blocks, (window + 63) / 64 + 1, a.rec32);
+    a.nsplit = prefill_splits(ws, ws_bytes, T, p0, window, true, n_q, blocks, a.rec32);
     a.part = (float*)ws;
     a.relu2 = false; a.scale32 = false; a.q_bf16 = dtype == EMBLA_BF16; a.out_bf16 = dtype == EMBLA_BF16;
     a.kring = (const uint16_t*)kring; a.vring = (const uint16_t*)vring; a.R = ring; a.qg = (const uint16_t*)qg;

@@ -86,3 +86,19 @@ def test_prefill_splits_precision(torch_gpu, T, p0):
         err.append(np.linalg.norm(f16_host(o) - ref) / np.linalg.norm(ref))
     print(f"[gpu-case] unsplit {err[0]:.3e} split {err[1]:.3e}", flush=True)
     assert err[1] <= 1.03 * err[0]
+
+
+@pytest.mark.parametrize("T,window", [(12, 1024), (193, 1024), (60, 4096)])
+def test_prefill_ring_without_a_prefix_is_one_pass(torch_gpu, T, window):
+    """A ring's splits follow the keys there are, not the window: a conversation's first message fills
+    a tile or two, and the call with a workspace is the unsplit one, bit for bit."""
+    from embla_attn import ops
+    torch = torch_gpu
+    R = (window + T + 127) // 128 * 128
+    say(f"prefill ring without a prefix T={T} window={window}")
+    g = torch.Generator("cuda").manual_seed(T)
+    k, v = (torch.randn(4 * R * 128, generator=g, device="cuda").half() for _ in range(2))
+    q = torch.randn(T, 16, 128, generator=g, device="cuda").half()
+    a, b = (ops.prefill_ring(q, k, v, T, 0, R, window, 4, dtype=ops.F16, ws=ws) for ws in (None, ops.PrefillWorkspace(T, 16)))
+    torch.cuda.synchronize()
+    assert torch.equal(a, b)
