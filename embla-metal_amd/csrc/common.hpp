@@ -151,7 +151,7 @@ __device__ __forceinline__ float max_rows(float v) { return fmax_xor32(max_xor16
 __device__ __forceinline__ float sum_rows(float v) { return sum_xor32(sum_xor16(v)); }
 /// DPP moves (VALU, no LDS round trip); CTRL: quad_perm 0xB1 (lane xor 1), 0x4E (xor 2),
 /// row_half_mirror 0x141 (lane 7 - i of its 8), row_mirror 0x140, row_shr:n 0x110 + n, row_ror:n
-/// 0x120 + n, row_bcast:15 0x142, row_bcast:31 0x143. Lanes with no source (bound_ctrl) and rows
+/// 0x120 + n, wave_shr:1 0x138, row_bcast:15 0x142, row_bcast:31 0x143. Lanes with no source (bound_ctrl) and rows
 /// off in ROW_MASK read 0.
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {

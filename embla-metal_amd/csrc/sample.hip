@@ -338,7 +338,9 @@ __global__ __launch_bounds__(FT) void sample_final_kernel(const uint16_t* __rest
         for (int o = 32; o >= 1; o >>= 1) small += __shfl_xor(small, o, 64);
         if (lane == 0) wsmall[t >> 6] = small;
         __syncthreads();
-        // thread t holds bins 4t .. 4t + 3, from the largest value down: their masses, scanned
+        // thread t holds bins 4t .. 4t + 3, from the largest value down: their masses, scanned. A bin
+        // starts at the very sum the one before it ends at, also across threads, so that one of them
+        // crosses want whatever the sums round to
         {
             const u4_t n4 = *(const u4_t*)&hist[4 * t];
             float eb[4];
@@ -360,15 +362,19 @@ __global__ __launch_bounds__(FT) void sample_final_kernel(const uint16_t* __rest
                 const double up = __shfl_up(incl, o, 64);
                 if (lane >= o) incl += up;
             }
+            const u2_t ib = __builtin_bit_cast(u2_t, incl);
+            const double prev = __builtin_bit_cast(double, (u2_t){dpp_u32<0x138>(ib[0]), dpp_u32<0x138>(ib[1])});   // wave_shr:1
             const int w = t >> 6;
             if (lane == 63) wtot[w] = incl;
             __syncthreads();
-            double before = incl - run;
+            double base = 0.0;
 #pragma unroll
-            for (int i = 0; i < FW; i++) before += i < w ? wtot[i] : 0.0;
+            for (int i = 0; i < FW; i++) base += i < w ? wtot[i] : 0.0;
+            double before = base + prev;   // (0 into lane 0)
+            const double end = base + incl;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                const double after = before + m4[k];
+                const double after = k == 3 ? end : fmin(before + m4[k], end);
                 if ((float)before < want && (float)after >= want) estar = 4 * t + k == CV_ZERO ? 2.0f : eb[k];
                 before = after;
             }
