@@ -24,11 +24,16 @@
 //    over all tokens. The kept mass only changes at the e of a capped value, and a capped value is
 //    a bf16 in [-15, 15]: the tokens are counted a value (3555 of them), the values' masses scanned
 //    from the top, and the 20 steps then compare their midpoints with the e at which the kept mass
-//    reaches top-p: the same decisions without a pass over the tokens a step. When all tokens are in
+//    reaches top-p: the same decisions without a pass over the tokens a step. Values under 2^-10 share
+//    a bin: where they are most of the tokens, or the mass is reached among them, the steps not decided
+//    by the bin's ends sum the kept mass itself (the candidates' four steps a round, a wave a midpoint;
+//    the row's a step at a time). Rows of few values are counted a run at a time. When all tokens are in
 //    play it draws again only the blocks whose winner over all tokens lies outside the nucleus. A
 //    65536-token row of logits N(0, 2²) in this kernel: 43 us with the steps summed over the row's e
 //    (64 a thread in registers, a barrier a step), 19.5 this way; what is left is the row's read by
-//    one workgroup and three more chains of barriers.
+//    one workgroup and three more chains of barriers. Logits and draw of 65536 tokens, the steps summed
+//    / this way: N(0, 2²) 51 / 28 us, one value 46 / 27.5 (72 with an add a token), ±15 46 / 36 (48),
+//    all 0 46 / 46 (60 with the count first), 1000 tokens at 0 17.3 / 17.7 (41).
 // Every value a later kernel needs is recomputed from the capped bf16 with the same rounded
 // operations (__fmul_rn, __fsub_rn: no contraction), so x and e agree bit for bit between kernels.
 #include "common.hpp"
@@ -144,7 +149,24 @@ __global__ __launch_bounds__(64) void argmax_final_kernel(const float* __restric
 }
 
 // ------------------------------------------------------------------ the draw
-struct BlockRec { float z, cm; uint32_t nc; float s; uint32_t si; float x; uint32_t pad[2]; };   // x: the winner's
+// Capped values a bin each: magnitudes from 2^-10 to 15 (the softcap's largest), positive and negative,
+// and one bin for the smaller ones; bin d counts down from 15.
+constexpr int CV_LO = 0x3A80, CV_N = 0x4170 - CV_LO + 1;   // bf16 bits of 2^-10 and 15
+constexpr int CV_ZERO = CV_N, CV_BINS = 2 * CV_N + 1;
+/// The bin of a capped value's bits, or -1 (a NaN).
+__device__ __forceinline__ int cv_bin(uint32_t c) {
+    const int m = (int)(c & 0x7FFF) - CV_LO;
+    if (m >= CV_N) return -1;
+    return m < 0 ? CV_ZERO : (c & 0x8000) ? CV_ZERO + 1 + m : CV_ZERO - 1 - m;
+}
+/// The capped value of bin d != CV_ZERO.
+__device__ __forceinline__ float cv_value(int d) {
+    return d < CV_ZERO ? bf2f((uint16_t)(CV_LO + CV_ZERO - 1 - d)) : bf2f((uint16_t)(0x8000 | (CV_LO + d - CV_ZERO - 1)));
+}
+
+/// A block's sums of e and of the candidates' e, its candidates, its winner (score, token, x), its tokens
+/// under 2^-10, and those of every fourth token whose capped value is their wave's first one's.
+struct BlockRec { float z, cm; uint32_t nc; float s; uint32_t si; float x; uint32_t small, alike; };
 
 /// the global max of x's scale: the largest block maximum (every wave computes it)
 __device__ __forceinline__ float global_max(const float* bmax, int G) {
@@ -158,7 +180,7 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(const uint16_t* __r
                                                              const float* __restrict__ bmax, int G, uint32_t key,
                                                              BlockRec* __restrict__ rec, uint32_t* __restrict__ cand) {
     __shared__ float sz[4], scm[4], ss[4];
-    __shared__ uint32_t sn[4], ssi[4];
+    __shared__ uint32_t sn[4], ssi[4], sl[4];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, b = blockIdx.x, i0 = b * SB + 4 * t;
     const float M = global_max(bmax, G);
     uint16_t c[4];
@@ -171,9 +193,11 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(const uint16_t* __r
     }
     float z = 0.0f, cm = 0.0f, best = NEG_INF;
     uint32_t n = 0, bi = 0xFFFFFFFFu, mine = 0;   // mine: bit k set for a candidate
+    const uint32_t alike = (uint32_t)__popcll(__ballot(i0 < V && c[0] == __builtin_amdgcn_readfirstlane(c[0])));
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         if (i0 + k >= V) continue;
+        if (cv_bin(c[k]) == CV_ZERO) n += 1u << 16;   // (above the candidates' count)
         const float x = __fsub_rn(__fmul_rn(bf2f(c[k]), inv_t), M);
         const float e = expf(x);
         z += e;
@@ -187,25 +211,27 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(const uint16_t* __r
     cm = wave_sum(cm);
     wave_best(best, bi);
     if (lane == 63) sn[w] = incl;
-    if (lane == 0) { sz[w] = z; scm[w] = cm; ss[w] = best; ssi[w] = bi; }
+    if (lane == 0) { sz[w] = z; scm[w] = cm; ss[w] = best; ssi[w] = bi; sl[w] = alike; }
     __syncthreads();
-    uint32_t at = incl - n;
-    for (int ww = 0; ww < w; ww++) at += sn[ww];
+    uint32_t at = (incl - n) & 0xFFFF;
+    for (int ww = 0; ww < w; ww++) at += sn[ww] & 0xFFFF;
     uint32_t* out = cand + (size_t)b * SB;
 #pragma unroll
     for (int k = 0; k < 4; k++)
         if (mine >> k & 1u) out[at++] = ((uint32_t)(i0 + k) << 16) | c[k];
     if (t == 0) {
         BlockRec r;
-        r.z = sz[0]; r.cm = scm[0]; r.nc = sn[0]; r.s = ss[0]; r.si = ssi[0];
+        r.z = sz[0]; r.cm = scm[0]; r.nc = sn[0]; r.s = ss[0]; r.si = ssi[0]; r.alike = sl[0];
         for (int ww = 1; ww < 4; ww++) {
             r.z += sz[ww];
             r.cm += scm[ww];
             r.nc += sn[ww];
+            r.alike += sl[ww];
             best_of(r.s, r.si, ss[ww], ssi[ww]);
         }
+        r.small = r.nc >> 16;
+        r.nc &= 0xFFFF;
         r.x = r.si < (uint32_t)V ? __fsub_rn(__fmul_rn(bf2f(cb[r.si]), inv_t), M) : NEG_INF;
-        r.pad[0] = r.pad[1] = 0;
         rec[b] = r;
     }
 }
@@ -213,23 +239,8 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(const uint16_t* __r
 constexpr int FT = 1024;              // threads of the final workgroup
 constexpr int FW = FT / 64;
 constexpr int FPT = 65536 / FT;       // tokens a thread holds on the all-token path
-
-// Capped values a bin each: magnitudes from 2^-10 to 15 (the softcap's largest), positive and negative,
-// and one bin for the smaller ones; bin d counts down from 15.
-constexpr int CV_LO = 0x3A80, CV_N = 0x4170 - CV_LO + 1;   // bf16 bits of 2^-10 and 15
-constexpr int CV_ZERO = CV_N, CV_BINS = 2 * CV_N + 1;
 static_assert(SB == FT, "a token of a block a thread");
 static_assert(CV_BINS <= 4 * FT, "four bins a thread");
-/// The bin of a capped value's bits, or -1 (a NaN).
-__device__ __forceinline__ int cv_bin(uint32_t c) {
-    const int m = (int)(c & 0x7FFF) - CV_LO;
-    if (m >= CV_N) return -1;
-    return m < 0 ? CV_ZERO : (c & 0x8000) ? CV_ZERO + 1 + m : CV_ZERO - 1 - m;
-}
-/// The capped value of bin d != CV_ZERO.
-__device__ __forceinline__ float cv_value(int d) {
-    return d < CV_ZERO ? bf2f((uint16_t)(CV_LO + CV_ZERO - 1 - d)) : bf2f((uint16_t)(0x8000 | (CV_LO + d - CV_ZERO - 1)));
-}
 
 /// block-wide sum, every thread getting the same value; buf is FW floats, the caller alternates
 /// two buffers between calls so one barrier a call suffices
@@ -263,6 +274,7 @@ __global__ __launch_bounds__(FT) void sample_final_kernel(const uint16_t* __rest
     __shared__ float bv[FW];
     __shared__ uint32_t bix[FW];
     __shared__ float tot[3];
+    __shared__ uint32_t kinds[2];        // tokens under 2^-10, of every fourth those like their wave's first
     __shared__ float ws_[64], wx_[64];   // the blocks' all-token Gumbel winners: score, x
     __shared__ uint32_t wi_[64];
     __shared__ __attribute__((aligned(16))) uint32_t hist[4 * FT];   // tokens a capped value
@@ -287,7 +299,9 @@ __global__ __launch_bounds__(FT) void sample_final_kernel(const uint16_t* __rest
         wx_[lane] = lane < G ? r.x : NEG_INF;
         wave_best(s, si);
         const float z = wave_sum(lane < G ? r.z : 0.0f), cm = wave_sum(lane < G ? r.cm : 0.0f);
+        const uint32_t sa = wave_scan_incl(lane < G ? r.small | (r.alike << 17) : 0);   // at most 2^16, 2^14
         if (lane == 0) { tot[0] = z; tot[1] = cm; tot[2] = s; bix[0] = si; }
+        if (lane == 63) { kinds[0] = sa & 0x1FFFF; kinds[1] = sa >> 17; }
     }
     __syncthreads();
     const float z = tot[0], cm = tot[1];
@@ -297,11 +311,30 @@ __global__ __launch_bounds__(FT) void sample_final_kernel(const uint16_t* __rest
         const float want = __fmul_rn(top_p, z);
         float hi = 1.0f;
         const bool few = nc <= (uint32_t)NCAND && cm >= want;   // uniform: over the candidates alone
+        // tokens mostly under 2^-10, which the bins do not tell apart, are not worth counting
+        const bool count_it = 2 * kinds[0] <= (uint32_t)V || (few && 2 * nc <= (uint32_t)V);
         double small = 0.0;   // the mass of this thread's values under 2^-10
+        auto x_of = [&](uint32_t c) { return __fsub_rn(__fmul_rn(bf2f((uint16_t)c), inv_t), M); };
         auto count = [&](uint32_t c) {
             const int d = cv_bin(c);
-            if (d == CV_ZERO) small += (double)expf(__fsub_rn(__fmul_rn(bf2f((uint16_t)c), inv_t), M));
+            if (d == CV_ZERO) small += (double)expf(x_of(c));
             else if (d >= 0) atomicAdd(&hist[d], 1u);
+        };
+        // the same for rows of few values (saturated ones), whose adds would queue at a few words: one
+        // add for a thread's run of tokens alike
+        int run = -1;
+        uint32_t len = 0;
+        auto count_runs = [&](uint32_t c) {
+            const int d = cv_bin(c);
+            if (d == CV_ZERO) small += (double)expf(x_of(c));
+            else if (d >= 0) {
+                if (d != run) {
+                    if (len) atomicAdd(&hist[run], len);
+                    run = d;
+                    len = 0;
+                }
+                len++;
+            }
         };
         // every token on the other path: token 4 t + 4096 q + k
         auto quad = [&](int q) {
@@ -312,6 +345,7 @@ __global__ __launch_bounds__(FT) void sample_final_kernel(const uint16_t* __rest
             for (int k = 0; k < 4; k++) h[k] = i0 + k < V ? cb[i0 + k] : 0x7FC0;   // (a NaN: not counted)
             return (u2_t){h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
         };
+        float* ce = (float*)hist;   // the candidates' e, where no counts are (any more)
         if (few) {
             // gather the candidates: slot j belongs to the block whose range of off holds it
             for (uint32_t j = t; j < nc; j += FT) {
@@ -322,26 +356,36 @@ __global__ __launch_bounds__(FT) void sample_final_kernel(const uint16_t* __rest
                 }
                 const uint32_t wd = cand[(size_t)b0 * SB + (j - off[b0])];
                 cw[j] = wd;
-                count(wd & 0xFFFF);
+                if (count_it) count(wd & 0xFFFF);
+                else ce[j] = expf(x_of(wd & 0xFFFF));   // (the rest of hist stays 0)
             }
             lo = CMIN;
-        } else {
+        } else if (count_it) {
             u2_t c2[FPT / 4];
 #pragma unroll
             for (int q = 0; q < FPT / 4; q++) c2[q] = quad(q);
+            auto all = [&](auto one) {
 #pragma unroll
-            for (int q = 0; q < FPT / 4; q++)
+                for (int q = 0; q < FPT / 4; q++)
 #pragma unroll
-                for (int k = 0; k < 4; k++) count((c2[q][k >> 1] >> (16 * (k & 1))) & 0xFFFF);
+                    for (int k = 0; k < 4; k++) one((c2[q][k >> 1] >> (16 * (k & 1))) & 0xFFFF);
+            };
+            if (12 * kinds[1] > (uint32_t)V) {   // (of every fourth token)
+                all(count_runs);
+                if (len) atomicAdd(&hist[run], len);
+            } else {
+                all(count);
+            }
         }
+        int done = 0;   // bisection steps decided
+        if (count_it) {
 #pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) small += __shfl_xor(small, o, 64);
-        if (lane == 0) wsmall[t >> 6] = small;
-        __syncthreads();
-        // thread t holds bins 4t .. 4t + 3, from the largest value down: their masses, scanned. A bin
-        // starts at the very sum the one before it ends at, also across threads, so that one of them
-        // crosses want whatever the sums round to
-        {
+            for (int o = 32; o >= 1; o >>= 1) small += __shfl_xor(small, o, 64);
+            if (lane == 0) wsmall[t >> 6] = small;
+            __syncthreads();
+            // thread t holds bins 4t .. 4t + 3, from the largest value down: their masses, scanned. A
+            // bin starts at the very sum the one before it ends at, also across threads, so that one of
+            // them crosses want whatever the sums round to
             const u4_t n4 = *(const u4_t*)&hist[4 * t];
             float eb[4];
             double m4[4], run = 0.0;
@@ -379,15 +423,60 @@ __global__ __launch_bounds__(FT) void sample_final_kernel(const uint16_t* __rest
                 before = after;
             }
             __syncthreads();
-        }
-        if (estar != 2.0f) {
-            for (int it = 0; it < 20; it++) {   // the steps' decisions: kept >= want up to that e
-                const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
-                if (mid <= estar) lo = mid; else hi = mid;
+            if (estar != 2.0f) {
+                for (; done < 20; done++) {   // the steps' decisions: kept >= want up to that e
+                    const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
+                    if (mid <= estar) lo = mid; else hi = mid;
+                }
+            } else {   // among the values under 2^-10: the steps whose midpoint lies outside the bin's e
+                const float e_lo = expf(x_of(0x8000 | (CV_LO - 1))) * (1.0f - 0x1p-20f);   // (room for expf's last bits)
+                const float e_hi = expf(x_of(CV_LO - 1)) * (1.0f + 0x1p-20f);
+                for (; done < 20; done++) {
+                    const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
+                    if (mid > e_lo && mid <= e_hi) break;
+                    if (mid <= e_lo) lo = mid; else hi = mid;
+                }
             }
-        } else {
-            // the mass is reached among the values under 2^-10, not told apart above: step by step, over
-            // the row's e in registers (64 a thread; candidates are all that a midpoint above CMIN keeps)
+        }
+        if (done < 20 && few) {
+            // the rest four steps a round: wave w = 1 .. 15 sums the kept mass at node w of the next four
+            // levels' decision tree (heap order; a passed step goes to child 2w + 1), then every thread
+            // walks the levels
+            const int w = t >> 6;
+            if (count_it)
+                for (uint32_t j = t; j < (uint32_t)NCAND; j += FT) ce[j] = j < nc ? expf(x_of(cw[j] & 0xFFFF)) : 0.0f;
+            __syncthreads();
+            float ev[NCAND / 64];
+#pragma unroll
+            for (int k = 0; k < NCAND / 64; k++) ev[k] = ce[64 * k + lane];
+            for (int r = 0; done < 20; r++) {
+                if (w >= 1) {
+                    float l2 = lo, h2 = hi;
+                    for (int d = 30 - __clz(w); d >= 0; d--) {   // the path's decisions: the bits of w below its top
+                        const float m = __fmul_rn(0.5f, __fadd_rn(l2, h2));
+                        if ((w >> d) & 1) l2 = m; else h2 = m;
+                    }
+                    const float mid = __fmul_rn(0.5f, __fadd_rn(l2, h2));
+                    float kept = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < NCAND / 64; k++) kept += ev[k] >= mid ? ev[k] : 0.0f;
+                    kept = wave_sum(kept);
+                    if (lane == 0) red[r & 1][w] = kept;
+                }
+                __syncthreads();
+                int node = 1;
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    if (done == 20) break;   // uniform
+                    const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
+                    const bool pass = red[r & 1][node] >= want;
+                    if (pass) lo = mid; else hi = mid;
+                    node = 2 * node + (pass ? 1 : 0);
+                    done++;
+                }
+            }
+        } else if (done < 20) {
+            // step by step over the row's e in registers (64 a thread)
             float e[FPT];
 #pragma unroll
             for (int q = 0; q < FPT / 4; q++) {
@@ -395,16 +484,15 @@ __global__ __launch_bounds__(FT) void sample_final_kernel(const uint16_t* __rest
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     const int i = 4 * t + 4 * FT * q + k;
-                    const uint16_t c = (uint16_t)(c2[k >> 1] >> (16 * (k & 1)));
-                    e[4 * q + k] = i < V ? expf(__fsub_rn(__fmul_rn(bf2f(c), inv_t), M)) : 0.0f;
+                    e[4 * q + k] = i < V ? expf(x_of((c2[k >> 1] >> (16 * (k & 1))) & 0xFFFF)) : 0.0f;
                 }
             }
-            for (int it = 0; it < 20; it++) {
+            for (; done < 20; done++) {
                 const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
                 float kept = 0.0f;
 #pragma unroll
                 for (int k = 0; k < FPT; k++) kept += e[k] >= mid ? e[k] : 0.0f;
-                if (block_sum(kept, red[it & 1]) >= want) lo = mid; else hi = mid;
+                if (block_sum(kept, red[done & 1]) >= want) lo = mid; else hi = mid;
             }
         }
         if (few) {

@@ -74,6 +74,10 @@ def logits_row(seed, V, kind, a):
         return lg
     if kind == "normal":
         return (g.standard_normal(V) * a).astype(np.float32)
+    if kind == "saturated":   # a share `a` at the softcap's 15, the rest at -15
+        return np.where(g.random(V) < a, 900.0, -900.0).astype(np.float32)
+    if kind == "mixed":   # a share `a` at one of two values under 2^-10, the rest at one of three above it
+        return np.where(g.random(V) < a, g.choice([-0.0009, 0.0009], V), g.choice([-1.0, 0.5, 1.0], V)).astype(np.float32)
     lg = (g.standard_normal(V) - 6).astype(np.float32)
     hot = g.choice(V, int(a), replace=False)
     lg[hot] = g.uniform(2, 8, int(a)).astype(np.float32)
@@ -93,6 +97,11 @@ CASES = [  # (seed, V, kind, a, T, top_p)
     # the mass reached among capped values under 2^-10, and just above them
     (13, 65536, "two", 0.6, 1.0, 0.3), (14, 30000, "two", 0.6, 0.8, 0.9), (15, 1500, "two", 0.7, 1.0, 0.5),
     (16, 65536, "normal", 0.004, 1.0, 0.95), (17, 2000, "normal", 2.5, 1.0, 0.9), (18, 7, "normal", 1.0, 1.0, 0.5),
+    # rows of one value or two, mostly under 2^-10, and of few values above it
+    (19, 65536, "saturated", 1.0, 1.0, 0.9), (20, 65533, "saturated", 0.3, 1.0, 0.9), (21, 2100, "saturated", 1.0, 1.3, 0.5),
+    (22, 1000, "saturated", 1.0, 1.0, 0.9), (23, 65536, "mixed", 0.4, 1.0, 0.9), (24, 30000, "mixed", 0.45, 1.0, 0.6),
+    (25, 65536, "mixed", 0.8, 1.0, 0.75), (26, 1500, "mixed", 0.9, 1.0, 0.4), (27, 1500, "mixed", 0.3, 0.9, 0.8),
+    (28, 65536, "normal", 2e-4, 1.0, 0.9), (29, 1000, "two", 0.6, 0.05, 0.9), (30, 65536, "mixed", 0.1, 1.0, 0.95),
 ]
 
 
