@@ -241,16 +241,20 @@ __global__ __launch_bounds__(256) void gemv_q4_rows_kernel(GemvArgs a) {
 }
 
 // Rows of one segment from which gemv_q4_rows_kernel takes over, and its workgroups at most (us, a row
-// a wave / this; K = 2048): 2048 rows 3.13 / 3.61, 3072 3.71 / 3.75, 4096 3.98 / 3.79, 8192 5.77 /
-// 4.83, 16384 8.54 / 6.57, 65536 24.7 / 16.3-17.5; K = 4096: 3072 5.23 / 5.04, 65536 40.3 / 28.7. 2048
-// workgroups were no faster at 65536 rows (16.4) and slower below (16384: 9.6), 4 rows a wave 17.2.
+// a wave / this; fp32 outputs; K = 2048): 2048 rows 3.13 / 3.61, 3072 3.71 / 3.75, 4096 3.56 / 3.36,
+// 8192 4.88 / 3.89, 16384 7.84 / 5.55, 65536 23.8 / 14.9; K = 4096: 3072 5.23 / 5.04, 65536 39.2 / 25.5.
+// 2048 workgroups were no faster at 65536 rows and slower below (16384: 9.6), 4 rows a wave 17.2.
 constexpr int GEMV_MANY_ROWS = 4096, GEMV_WG = 1024;
 
 template <int EPI>
 void launch_gemv_q4_epi(const GemvArgs& a, hipStream_t st) {
     const int rows = (int)a.seg[a.nseg - 1].end;
     if (a.nseg == 1 && rows >= GEMV_MANY_ROWS) {
-        const dim3 grid(min(rows / (8 * GEMV_RW), GEMV_WG));
+        // a workgroup's turn is two loads of its 4 waves' rows. Rows past the last whole turn take a turn more
+        // of a few workgroups, or up to two workgroups a CU one more workgroup (4200 rows: 3.95 us a row a
+        // wave, 4.15 with 262 workgroups, 3.77 with 263; 8200 rows of 4096: 7.7, 6.3 with 512, 6.7 with 513)
+        constexpr int TURN = 8 * GEMV_RW;
+        const dim3 grid(min((rows + (rows < 512 * TURN ? TURN - 1 : 0)) / TURN, GEMV_WG));
         if (a.K == 2048) hipLaunchKernelGGL((gemv_q4_rows_kernel<EPI, 1>), grid, dim3(256), 0, st, a);
         else hipLaunchKernelGGL((gemv_q4_rows_kernel<EPI, 2>), grid, dim3(256), 0, st, a);
     } else {
