@@ -25,15 +25,15 @@
 //    a bf16 in [-15, 15]: the tokens are counted a value (3555 of them), the values' masses scanned
 //    from the top, and the 20 steps then compare their midpoints with the e at which the kept mass
 //    reaches top-p: the same decisions without a pass over the tokens a step. Values under 2^-10 share
-//    a bin: where they are most of the tokens, or the mass is reached among them, the steps not decided
-//    by the bin's ends sum the kept mass itself (the candidates' four steps a round, a wave a midpoint;
-//    the row's a step at a time). Rows of few values are counted a run at a time. When all tokens are in
-//    play it draws again only the blocks whose winner over all tokens lies outside the nucleus. A
-//    65536-token row of logits N(0, 2²) in this kernel: 43 us with the steps summed over the row's e
-//    (64 a thread in registers, a barrier a step), 19.5 this way; what is left is the row's read by
-//    one workgroup and three more chains of barriers. Logits and draw of 65536 tokens, the steps summed
-//    / this way: N(0, 2²) 51 / 28 us, one value 46 / 27.5 (72 with an add a token), ±15 46 / 36 (48),
-//    all 0 46 / 46 (60 with the count first), 1000 tokens at 0 17.3 / 17.7 (41).
+//    a bin: where the mass is reached among them (the blocks' sums of e down to the bin's ends tell),
+//    nothing is counted and the steps sum the kept mass itself (the candidates' four steps a round, a
+//    wave a midpoint; the row's a step at a time). Rows of few values are counted a run at a time.
+//    When all tokens are in play it draws again only the blocks whose winner over all tokens lies
+//    outside the nucleus. What bounds it: the row's read by one workgroup, and the chain of five barriers
+//    around the count. Draws of 65536 tokens at top-p 0.9, the steps summed over the row's e (64 a thread
+//    in registers, a barrier a step) / this way, with the two kernels before: N(0, 2²) 52.0 / 29.8 us,
+//    one value 47.0 / 28.3 (72.7 with an add a token), ±15 46.8 / 36.6, all 0 46.6 / 45.8 (60.5 counted
+//    first); at top-p 0.5 N(0, 0.002²) 57.6 / 58.3 (67.3 counted first); 2000 tokens 19.6 / 17.6.
 // Every value a later kernel needs is recomputed from the capped bf16 with the same rounded
 // operations (__fmul_rn, __fsub_rn: no contraction), so x and e agree bit for bit between kernels.
 #include "common.hpp"
@@ -164,9 +164,10 @@ __device__ __forceinline__ float cv_value(int d) {
     return d < CV_ZERO ? bf2f((uint16_t)(CV_LO + CV_ZERO - 1 - d)) : bf2f((uint16_t)(0x8000 | (CV_LO + d - CV_ZERO - 1)));
 }
 
-/// A block's sums of e and of the candidates' e, its candidates, its winner (score, token, x), its tokens
-/// under 2^-10, and those of every fourth token whose capped value is their wave's first one's.
-struct BlockRec { float z, cm; uint32_t nc; float s; uint32_t si; float x; uint32_t small, alike; };
+/// A block's sums of e: all tokens', the candidates', those of values from 2^-10 up and above -2^-10 (the
+/// kept mass at the ends of the small values' bin); its winner (score, token, x); its candidates, and above
+/// them (<< 16) those of every fourth token whose capped value is their wave's first one's (from 2^-10 up).
+struct BlockRec { float z, cm, up, low, s; uint32_t si; float x; uint32_t n; };
 
 /// the global max of x's scale: the largest block maximum (every wave computes it)
 __device__ __forceinline__ float global_max(const float* bmax, int G) {
@@ -179,8 +180,8 @@ __device__ __forceinline__ float global_max(const float* bmax, int G) {
 __global__ __launch_bounds__(256) void sample_weights_kernel(const uint16_t* __restrict__ cb, int V, float inv_t,
                                                              const float* __restrict__ bmax, int G, uint32_t key,
                                                              BlockRec* __restrict__ rec, uint32_t* __restrict__ cand) {
-    __shared__ float sz[4], scm[4], ss[4];
-    __shared__ uint32_t sn[4], ssi[4], sl[4];
+    __shared__ float sz[4], scm[4], su[4], sl[4], ss[4];
+    __shared__ uint32_t sn[4], ssi[4];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, b = blockIdx.x, i0 = b * SB + 4 * t;
     const float M = global_max(bmax, G);
     uint16_t c[4];
@@ -191,16 +192,18 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(const uint16_t* __r
 #pragma unroll
         for (int k = 0; k < 4; k++) c[k] = i0 + k < V ? cb[i0 + k] : 0;
     }
-    float z = 0.0f, cm = 0.0f, best = NEG_INF;
+    float z = 0.0f, cm = 0.0f, up = 0.0f, low = 0.0f, best = NEG_INF;
     uint32_t n = 0, bi = 0xFFFFFFFFu, mine = 0;   // mine: bit k set for a candidate
-    const uint32_t alike = (uint32_t)__popcll(__ballot(i0 < V && c[0] == __builtin_amdgcn_readfirstlane(c[0])));
+    const uint32_t alike = (uint32_t)__popcll(__ballot(i0 < V && c[0] == __builtin_amdgcn_readfirstlane(c[0]) &&
+                                                       cv_bin(c[0]) != CV_ZERO));
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         if (i0 + k >= V) continue;
-        if (cv_bin(c[k]) == CV_ZERO) n += 1u << 16;   // (above the candidates' count)
         const float x = __fsub_rn(__fmul_rn(bf2f(c[k]), inv_t), M);
         const float e = expf(x);
         z += e;
+        up += bf2f(c[k]) >= 0x1p-10f ? e : 0.0f;
+        low += bf2f(c[k]) > -0x1p-10f ? e : 0.0f;
         if (e >= CMIN) { cm += e; n++; mine |= 1u << k; }
         best_of(best, bi, gumbel_score(x, key, (uint32_t)(i0 + k)), (uint32_t)(i0 + k));
     }
@@ -209,11 +212,13 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(const uint16_t* __r
     incl = wave_scan_incl(incl);
     z = wave_sum(z);
     cm = wave_sum(cm);
+    up = wave_sum(up);
+    low = wave_sum(low);
     wave_best(best, bi);
-    if (lane == 63) sn[w] = incl;
-    if (lane == 0) { sz[w] = z; scm[w] = cm; ss[w] = best; ssi[w] = bi; sl[w] = alike; }
+    if (lane == 63) sn[w] = incl | (alike << 16);
+    if (lane == 0) { sz[w] = z; scm[w] = cm; su[w] = up; sl[w] = low; ss[w] = best; ssi[w] = bi; }
     __syncthreads();
-    uint32_t at = (incl - n) & 0xFFFF;
+    uint32_t at = incl - n;
     for (int ww = 0; ww < w; ww++) at += sn[ww] & 0xFFFF;
     uint32_t* out = cand + (size_t)b * SB;
 #pragma unroll
@@ -221,16 +226,15 @@ __global__ __launch_bounds__(256) void sample_weights_kernel(const uint16_t* __r
         if (mine >> k & 1u) out[at++] = ((uint32_t)(i0 + k) << 16) | c[k];
     if (t == 0) {
         BlockRec r;
-        r.z = sz[0]; r.cm = scm[0]; r.nc = sn[0]; r.s = ss[0]; r.si = ssi[0]; r.alike = sl[0];
+        r.z = sz[0]; r.cm = scm[0]; r.up = su[0]; r.low = sl[0]; r.n = sn[0]; r.s = ss[0]; r.si = ssi[0];
         for (int ww = 1; ww < 4; ww++) {
             r.z += sz[ww];
             r.cm += scm[ww];
-            r.nc += sn[ww];
-            r.alike += sl[ww];
+            r.up += su[ww];
+            r.low += sl[ww];
+            r.n += sn[ww];
             best_of(r.s, r.si, ss[ww], ssi[ww]);
         }
-        r.small = r.nc >> 16;
-        r.nc &= 0xFFFF;
         r.x = r.si < (uint32_t)V ? __fsub_rn(__fmul_rn(bf2f(cb[r.si]), inv_t), M) : NEG_INF;
         rec[b] = r;
     }
@@ -273,270 +277,272 @@ __global__ __launch_bounds__(FT) void sample_final_kernel(const uint16_t* __rest
     __shared__ float red[2][FW];
     __shared__ float bv[FW];
     __shared__ uint32_t bix[FW];
-    __shared__ float tot[3];
-    __shared__ uint32_t kinds[2];        // tokens under 2^-10, of every fourth those like their wave's first
+    __shared__ float tot[4];             // the sums of z, cm, up, low
+    __shared__ uint32_t likes;           // of every fourth token those like their wave's first
     __shared__ float ws_[64], wx_[64];   // the blocks' all-token Gumbel winners: score, x
     __shared__ uint32_t wi_[64];
     __shared__ __attribute__((aligned(16))) uint32_t hist[4 * FT];   // tokens a capped value
     __shared__ double wtot[FW], wsmall[FW];
     __shared__ float estar;   // the e at which the kept mass reaches top-p (-1: nowhere; 2: in the bin of small values)
     const int t = threadIdx.x, lane = t & 63;
+    if (!(top_p < 1.0f)) {   // every token is in the nucleus: the best block winner
+        if (t < 64) {
+            float s = lane < G ? rec[lane].s : NEG_INF;
+            uint32_t si = lane < G ? rec[lane].si : 0xFFFFFFFFu;
+            wave_best(s, si);
+            if (lane == 0) write_token(si, token, greedy, pos, prompt);
+        }
+        return;
+    }
     const float M = global_max(bmax, G);
     *(u4_t*)&hist[4 * t] = (u4_t){0, 0, 0, 0};
     if (t == 0) estar = -1.0f;
-    // the block records: wave 0 sums them and scans the candidate counts
-    if (t < 64) {
+    // the block records: wave 0 scans the candidate counts, wave 1 sums the masses, wave 2 finds the best winner
+    if (t < 192) {
         BlockRec r = {};
         if (lane < G) r = rec[lane];
-        uint32_t incl = lane < G ? r.nc : 0;
-        incl = wave_scan_incl(incl);
-        off[lane + 1] = incl;
-        if (lane == 0) off[0] = 0;
-        float s = lane < G ? r.s : NEG_INF;
-        uint32_t si = lane < G ? r.si : 0xFFFFFFFFu;
-        ws_[lane] = s;
-        wi_[lane] = si;
-        wx_[lane] = lane < G ? r.x : NEG_INF;
-        wave_best(s, si);
-        const float z = wave_sum(lane < G ? r.z : 0.0f), cm = wave_sum(lane < G ? r.cm : 0.0f);
-        const uint32_t sa = wave_scan_incl(lane < G ? r.small | (r.alike << 17) : 0);   // at most 2^16, 2^14
-        if (lane == 0) { tot[0] = z; tot[1] = cm; tot[2] = s; bix[0] = si; }
-        if (lane == 63) { kinds[0] = sa & 0x1FFFF; kinds[1] = sa >> 17; }
+        if (t < 64) {
+            const uint32_t incl = wave_scan_incl((r.n & 0xFFFF) | (r.n >> 16 << 17));   // at most 2^16, 2^14
+            off[lane + 1] = incl & 0x1FFFF;
+            if (lane == 0) off[0] = 0;
+            ws_[lane] = r.s;
+            wi_[lane] = r.si;
+            wx_[lane] = r.x;
+            if (lane == 63) likes = incl >> 17;
+        } else if (t < 128) {
+            const float z = wave_sum(r.z), cm = wave_sum(r.cm), up = wave_sum(r.up), low = wave_sum(r.low);
+            if (lane == 0) { tot[0] = z; tot[1] = cm; tot[2] = up; tot[3] = low; }
+        } else {
+            float s = lane < G ? r.s : NEG_INF;
+            uint32_t si = lane < G ? r.si : 0xFFFFFFFFu;
+            wave_best(s, si);
+            if (lane == 0) bix[0] = si;
+        }
     }
     __syncthreads();
     const float z = tot[0], cm = tot[1];
     const uint32_t nc = off[G];
     float lo = 0.0f;
-    if (top_p < 1.0f) {
-        const float want = __fmul_rn(top_p, z);
-        float hi = 1.0f;
-        const bool few = nc <= (uint32_t)NCAND && cm >= want;   // uniform: over the candidates alone
-        // tokens mostly under 2^-10, which the bins do not tell apart, are not worth counting
-        const bool count_it = 2 * kinds[0] <= (uint32_t)V || (few && 2 * nc <= (uint32_t)V);
-        double small = 0.0;   // the mass of this thread's values under 2^-10
-        auto x_of = [&](uint32_t c) { return __fsub_rn(__fmul_rn(bf2f((uint16_t)c), inv_t), M); };
-        auto count = [&](uint32_t c) {
-            const int d = cv_bin(c);
-            if (d == CV_ZERO) small += (double)expf(x_of(c));
-            else if (d >= 0) atomicAdd(&hist[d], 1u);
-        };
-        // the same for rows of few values (saturated ones), whose adds would queue at a few words: one
-        // add for a thread's run of tokens alike
-        int run = -1;
-        uint32_t len = 0;
-        auto count_runs = [&](uint32_t c) {
-            const int d = cv_bin(c);
-            if (d == CV_ZERO) small += (double)expf(x_of(c));
-            else if (d >= 0) {
-                if (d != run) {
-                    if (len) atomicAdd(&hist[run], len);
-                    run = d;
-                    len = 0;
-                }
-                len++;
-            }
-        };
-        // every token on the other path: token 4 t + 4096 q + k
-        auto quad = [&](int q) {
-            const int i0 = 4 * t + 4 * FT * q;
-            if (i0 + 3 < V) return ld8(cb + i0);
-            uint32_t h[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) h[k] = i0 + k < V ? cb[i0 + k] : 0x7FC0;   // (a NaN: not counted)
-            return (u2_t){h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-        };
-        float* ce = (float*)hist;   // the candidates' e, where no counts are (any more)
-        if (few) {
-            // gather the candidates: slot j belongs to the block whose range of off holds it
-            for (uint32_t j = t; j < nc; j += FT) {
-                int b0 = 0, b1 = G - 1;   // last block with off[b] <= j
-                while (b0 < b1) {
-                    const int mid = (b0 + b1 + 1) >> 1;
-                    if (off[mid] <= j) b0 = mid; else b1 = mid - 1;
-                }
-                const uint32_t wd = cand[(size_t)b0 * SB + (j - off[b0])];
-                cw[j] = wd;
-                if (count_it) count(wd & 0xFFFF);
-                else ce[j] = expf(x_of(wd & 0xFFFF));   // (the rest of hist stays 0)
-            }
-            lo = CMIN;
-        } else if (count_it) {
-            u2_t c2[FPT / 4];
-#pragma unroll
-            for (int q = 0; q < FPT / 4; q++) c2[q] = quad(q);
-            auto all = [&](auto one) {
-#pragma unroll
-                for (int q = 0; q < FPT / 4; q++)
-#pragma unroll
-                    for (int k = 0; k < 4; k++) one((c2[q][k >> 1] >> (16 * (k & 1))) & 0xFFFF);
-            };
-            if (12 * kinds[1] > (uint32_t)V) {   // (of every fourth token)
-                all(count_runs);
+    const float want = __fmul_rn(top_p, z);
+    float hi = 1.0f;
+    const bool few = nc <= (uint32_t)NCAND && cm >= want;   // uniform: over the candidates alone
+    // the counts leave the steps undecided where the mass is reached among the values under 2^-10, which
+    // they do not tell apart: then they are not taken (either way the decisions are the same)
+    const bool count_it = !(tot[2] < want && want <= tot[3]);
+    double small = 0.0;   // the mass of this thread's values under 2^-10
+    auto x_of = [&](uint32_t c) { return __fsub_rn(__fmul_rn(bf2f((uint16_t)c), inv_t), M); };
+    auto count = [&](uint32_t c) {
+        const int d = cv_bin(c);
+        if (d == CV_ZERO) small += (double)expf(x_of(c));
+        else if (d >= 0) atomicAdd(&hist[d], 1u);
+    };
+    // the same for rows of few values (saturated ones), whose adds would queue at a few words: one
+    // add for a thread's run of tokens alike
+    int run = -1;
+    uint32_t len = 0;
+    auto count_runs = [&](uint32_t c) {
+        const int d = cv_bin(c);
+        if (d == CV_ZERO) small += (double)expf(x_of(c));
+        else if (d >= 0) {
+            if (d != run) {
                 if (len) atomicAdd(&hist[run], len);
-            } else {
-                all(count);
+                run = d;
+                len = 0;
             }
+            len++;
         }
-        int done = 0;   // bisection steps decided
-        if (count_it) {
+    };
+    // every token on the other path: token 4 t + 4096 q + k
+    auto quad = [&](int q) {
+        const int i0 = 4 * t + 4 * FT * q;
+        if (i0 + 3 < V) return ld8(cb + i0);
+        uint32_t h[4];
 #pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) small += __shfl_xor(small, o, 64);
-            if (lane == 0) wsmall[t >> 6] = small;
-            __syncthreads();
-            // thread t holds bins 4t .. 4t + 3, from the largest value down: their masses, scanned. A
-            // bin starts at the very sum the one before it ends at, also across threads, so that one of
-            // them crosses want whatever the sums round to
-            const u4_t n4 = *(const u4_t*)&hist[4 * t];
-            float eb[4];
-            double m4[4], run = 0.0;
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int d = 4 * t + k;
-                eb[k] = expf(__fsub_rn(__fmul_rn(d < CV_BINS && d != CV_ZERO ? cv_value(d) : 0.0f, inv_t), M));
-                m4[k] = n4[k] ? (double)n4[k] * (double)eb[k] : 0.0;
-                if (d == CV_ZERO) {
-#pragma unroll
-                    for (int i = 0; i < FW; i++) m4[k] += wsmall[i];
-                }
-                run += m4[k];
+        for (int k = 0; k < 4; k++) h[k] = i0 + k < V ? cb[i0 + k] : 0x7FC0;   // (a NaN: not counted)
+        return (u2_t){h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+    };
+    float* ce = (float*)hist;   // the candidates' e, where no counts are (any more)
+    if (few) {
+        // gather the candidates: slot j belongs to the block whose range of off holds it
+        for (uint32_t j = t; j < nc; j += FT) {
+            int b0 = 0, b1 = G - 1;   // last block with off[b] <= j
+            while (b0 < b1) {
+                const int mid = (b0 + b1 + 1) >> 1;
+                if (off[mid] <= j) b0 = mid; else b1 = mid - 1;
             }
-            double incl = run;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const double up = __shfl_up(incl, o, 64);
-                if (lane >= o) incl += up;
-            }
-            const u2_t ib = __builtin_bit_cast(u2_t, incl);
-            const double prev = __builtin_bit_cast(double, (u2_t){dpp_u32<0x138>(ib[0]), dpp_u32<0x138>(ib[1])});   // wave_shr:1
-            const int w = t >> 6;
-            if (lane == 63) wtot[w] = incl;
-            __syncthreads();
-            double base = 0.0;
-#pragma unroll
-            for (int i = 0; i < FW; i++) base += i < w ? wtot[i] : 0.0;
-            double before = base + prev;   // (0 into lane 0)
-            const double end = base + incl;
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const double after = k == 3 ? end : fmin(before + m4[k], end);
-                if ((float)before < want && (float)after >= want) estar = 4 * t + k == CV_ZERO ? 2.0f : eb[k];
-                before = after;
-            }
-            __syncthreads();
-            if (estar != 2.0f) {
-                for (; done < 20; done++) {   // the steps' decisions: kept >= want up to that e
-                    const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
-                    if (mid <= estar) lo = mid; else hi = mid;
-                }
-            } else {   // among the values under 2^-10: the steps whose midpoint lies outside the bin's e
-                const float e_lo = expf(x_of(0x8000 | (CV_LO - 1))) * (1.0f - 0x1p-20f);   // (room for expf's last bits)
-                const float e_hi = expf(x_of(CV_LO - 1)) * (1.0f + 0x1p-20f);
-                for (; done < 20; done++) {
-                    const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
-                    if (mid > e_lo && mid <= e_hi) break;
-                    if (mid <= e_lo) lo = mid; else hi = mid;
-                }
-            }
+            const uint32_t wd = cand[(size_t)b0 * SB + (j - off[b0])];
+            cw[j] = wd;
+            if (count_it) count(wd & 0xFFFF);
+            else ce[j] = expf(x_of(wd & 0xFFFF));   // (the rest of hist stays 0)
         }
-        if (done < 20 && few) {
-            // the rest four steps a round: wave w = 1 .. 15 sums the kept mass at node w of the next four
-            // levels' decision tree (heap order; a passed step goes to child 2w + 1), then every thread
-            // walks the levels
-            const int w = t >> 6;
-            if (count_it)
-                for (uint32_t j = t; j < (uint32_t)NCAND; j += FT) ce[j] = j < nc ? expf(x_of(cw[j] & 0xFFFF)) : 0.0f;
-            __syncthreads();
-            float ev[NCAND / 64];
+        lo = CMIN;
+    } else if (count_it) {
+        u2_t c2[FPT / 4];
 #pragma unroll
-            for (int k = 0; k < NCAND / 64; k++) ev[k] = ce[64 * k + lane];
-            for (int r = 0; done < 20; r++) {
-                if (w >= 1) {
-                    float l2 = lo, h2 = hi;
-                    for (int d = 30 - __clz(w); d >= 0; d--) {   // the path's decisions: the bits of w below its top
-                        const float m = __fmul_rn(0.5f, __fadd_rn(l2, h2));
-                        if ((w >> d) & 1) l2 = m; else h2 = m;
-                    }
-                    const float mid = __fmul_rn(0.5f, __fadd_rn(l2, h2));
-                    float kept = 0.0f;
+        for (int q = 0; q < FPT / 4; q++) c2[q] = quad(q);
+        auto all = [&](auto one) {
 #pragma unroll
-                    for (int k = 0; k < NCAND / 64; k++) kept += ev[k] >= mid ? ev[k] : 0.0f;
-                    kept = wave_sum(kept);
-                    if (lane == 0) red[r & 1][w] = kept;
-                }
-                __syncthreads();
-                int node = 1;
+            for (int q = 0; q < FPT / 4; q++)
 #pragma unroll
-                for (int d = 0; d < 4; d++) {
-                    if (done == 20) break;   // uniform
-                    const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
-                    const bool pass = red[r & 1][node] >= want;
-                    if (pass) lo = mid; else hi = mid;
-                    node = 2 * node + (pass ? 1 : 0);
-                    done++;
-                }
+                for (int k = 0; k < 4; k++) one((c2[q][k >> 1] >> (16 * (k & 1))) & 0xFFFF);
+        };
+        if (12 * likes > (uint32_t)V) {   // (of every fourth token)
+            all(count_runs);
+            if (len) atomicAdd(&hist[run], len);
+        } else {
+            all(count);
+        }
+    }
+    bool decided = false;   // the bisection's steps
+    if (count_it) {
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) small += __shfl_xor(small, o, 64);
+        if (lane == 0) wsmall[t >> 6] = small;
+        __syncthreads();
+        // thread t holds bins 4t .. 4t + 3, from the largest value down: their masses, scanned. A
+        // bin starts at the very sum the one before it ends at, also across threads, so that one of
+        // them crosses want whatever the sums round to
+        const u4_t n4 = *(const u4_t*)&hist[4 * t];
+        float eb[4];
+        double m4[4], run = 0.0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int d = 4 * t + k;
+            eb[k] = expf(__fsub_rn(__fmul_rn(d < CV_BINS && d != CV_ZERO ? cv_value(d) : 0.0f, inv_t), M));
+            m4[k] = n4[k] ? (double)n4[k] * (double)eb[k] : 0.0;
+            if (d == CV_ZERO) {
+#pragma unroll
+                for (int i = 0; i < FW; i++) m4[k] += wsmall[i];
             }
-        } else if (done < 20) {
-            // step by step over the row's e in registers (64 a thread)
-            float e[FPT];
+            run += m4[k];
+        }
+        double incl = run;
 #pragma unroll
-            for (int q = 0; q < FPT / 4; q++) {
-                const u2_t c2 = quad(q);
+        for (int o = 1; o < 64; o <<= 1) {
+            const double up = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += up;
+        }
+        const u2_t ib = __builtin_bit_cast(u2_t, incl);
+        const double prev = __builtin_bit_cast(double, (u2_t){dpp_u32<0x138>(ib[0]), dpp_u32<0x138>(ib[1])});   // wave_shr:1
+        const int w = t >> 6;
+        if (lane == 63) wtot[w] = incl;
+        __syncthreads();
+        double base = 0.0;
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int i = 4 * t + 4 * FT * q + k;
-                    e[4 * q + k] = i < V ? expf(x_of((c2[k >> 1] >> (16 * (k & 1))) & 0xFFFF)) : 0.0f;
-                }
-            }
-            for (; done < 20; done++) {
+        for (int i = 0; i < FW; i++) base += i < w ? wtot[i] : 0.0;
+        double before = base + prev;   // (0 into lane 0)
+        const double end = base + incl;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const double after = k == 3 ? end : fmin(before + m4[k], end);
+            if ((float)before < want && (float)after >= want) estar = 4 * t + k == CV_ZERO ? 2.0f : eb[k];
+            before = after;
+        }
+        __syncthreads();
+        if (estar != 2.0f) {   // (2: the sums' rounding moved the crossing into the bin of small values)
+            for (int step = 0; step < 20; step++) {   // the steps' decisions: kept >= want up to that e
                 const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
+                if (mid <= estar) lo = mid; else hi = mid;
+            }
+            decided = true;
+        }
+    }
+    if (!decided && few) {
+        // four steps a round: wave w = 1 .. 15 sums the kept mass at node w of the next four
+        // levels' decision tree (heap order; a passed step goes to child 2w + 1), then every thread
+        // walks the levels
+        const int w = t >> 6;
+        if (count_it)
+            for (uint32_t j = t; j < (uint32_t)NCAND; j += FT) ce[j] = j < nc ? expf(x_of(cw[j] & 0xFFFF)) : 0.0f;
+        __syncthreads();
+        float ev[NCAND / 64];
+#pragma unroll
+        for (int k = 0; k < NCAND / 64; k++) ev[k] = ce[64 * k + lane];
+        for (int r = 0; r < 5; r++) {
+            if (w >= 1) {
+                float l2 = lo, h2 = hi;
+                for (int d = 30 - __clz(w); d >= 0; d--) {   // the path's decisions: the bits of w below its top
+                    const float m = __fmul_rn(0.5f, __fadd_rn(l2, h2));
+                    if ((w >> d) & 1) l2 = m; else h2 = m;
+                }
+                const float mid = __fmul_rn(0.5f, __fadd_rn(l2, h2));
                 float kept = 0.0f;
 #pragma unroll
-                for (int k = 0; k < FPT; k++) kept += e[k] >= mid ? e[k] : 0.0f;
-                if (block_sum(kept, red[done & 1]) >= want) lo = mid; else hi = mid;
+                for (int k = 0; k < NCAND / 64; k++) kept += ev[k] >= mid ? ev[k] : 0.0f;
+                kept = wave_sum(kept);
+                if (lane == 0) red[r & 1][w] = kept;
             }
-        }
-        if (few) {
-            const float floor_x = logf(lo);
-            float best = NEG_INF;
-            uint32_t bi = 0xFFFFFFFFu;
-            for (uint32_t j = t; j < nc; j += FT) {
-                const uint32_t wd = cw[j], i = wd >> 16;
-                const float x = __fsub_rn(__fmul_rn(bf2f((uint16_t)(wd & 0xFFFF)), inv_t), M);
-                if (x >= floor_x) best_of(best, bi, gumbel_score(x, key, i), i);
-            }
-            block_best(best, bi, bv, bix);
-            if (t == 0) write_token(bi, token, greedy, pos, prompt);
-            return;
-        }
-        if (lo > 0.0f) {
-            // a block's winner over all its tokens is its winner over its nucleus tokens when it is in
-            // the nucleus itself; the other blocks (a tenth at top-p 0.9) are drawn again, a token a
-            // thread, four blocks' loads in flight (a wave a block took its 16 tokens a lane in turn)
-            const float floor_x = logf(lo);
-            float best = NEG_INF;
-            uint32_t bi = 0xFFFFFFFFu;
-            const bool in = lane < G && wx_[lane] >= floor_x;
-            if (in) best_of(best, bi, ws_[lane], wi_[lane]);
-            uint64_t redo = __ballot(lane < G && !in);   // the same in every wave
-            while (redo) {
-                int i4[4];
-                uint16_t c4[4];
+            __syncthreads();
+            int node = 1;
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    i4[k] = redo ? (__ffsll((unsigned long long)redo) - 1) * SB + t : V;
-                    redo &= redo - 1;   // (0 stays 0)
-                    c4[k] = i4[k] < V ? cb[i4[k]] : 0x7FC0;
-                }
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const float x = __fsub_rn(__fmul_rn(bf2f(c4[k]), inv_t), M);
-                    if (i4[k] < V && x >= floor_x) best_of(best, bi, gumbel_score(x, key, (uint32_t)i4[k]), (uint32_t)i4[k]);
-                }
+            for (int d = 0; d < 4; d++) {
+                const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
+                const bool pass = red[r & 1][node] >= want;
+                if (pass) lo = mid; else hi = mid;
+                node = 2 * node + (pass ? 1 : 0);
             }
-            block_best(best, bi, bv, bix);
-            if (t == 0) write_token(bi, token, greedy, pos, prompt);
-            return;
         }
+    } else if (!decided) {
+        // step by step over the row's e in registers (64 a thread)
+        float e[FPT];
+#pragma unroll
+        for (int q = 0; q < FPT / 4; q++) {
+            const u2_t c2 = quad(q);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int i = 4 * t + 4 * FT * q + k;
+                e[4 * q + k] = i < V ? expf(x_of((c2[k >> 1] >> (16 * (k & 1))) & 0xFFFF)) : 0.0f;
+            }
+        }
+        for (int step = 0; step < 20; step++) {
+            const float mid = __fmul_rn(0.5f, __fadd_rn(lo, hi));
+            float kept = 0.0f;
+#pragma unroll
+            for (int k = 0; k < FPT; k++) kept += e[k] >= mid ? e[k] : 0.0f;
+            if (block_sum(kept, red[step & 1]) >= want) lo = mid; else hi = mid;
+        }
+    }
+    if (few) {
+        const float floor_x = logf(lo);
+        float best = NEG_INF;
+        uint32_t bi = 0xFFFFFFFFu;
+        for (uint32_t j = t; j < nc; j += FT) {
+            const uint32_t wd = cw[j], i = wd >> 16;
+            const float x = __fsub_rn(__fmul_rn(bf2f((uint16_t)(wd & 0xFFFF)), inv_t), M);
+            if (x >= floor_x) best_of(best, bi, gumbel_score(x, key, i), i);
+        }
+        block_best(best, bi, bv, bix);
+        if (t == 0) write_token(bi, token, greedy, pos, prompt);
+        return;
+    }
+    if (lo > 0.0f) {
+        // a block's winner over all its tokens is its winner over its nucleus tokens when it is in
+        // the nucleus itself; the other blocks (a tenth at top-p 0.9) are drawn again, a token a
+        // thread, four blocks' loads in flight (a wave a block took its 16 tokens a lane in turn)
+        const float floor_x = logf(lo);
+        float best = NEG_INF;
+        uint32_t bi = 0xFFFFFFFFu;
+        const bool in = lane < G && wx_[lane] >= floor_x;
+        if (in) best_of(best, bi, ws_[lane], wi_[lane]);
+        uint64_t redo = __ballot(lane < G && !in);   // the same in every wave
+        while (redo) {
+            int i4[4];
+            uint16_t c4[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                i4[k] = redo ? (__ffsll((unsigned long long)redo) - 1) * SB + t : V;
+                redo &= redo - 1;   // (0 stays 0)
+                c4[k] = i4[k] < V ? cb[i4[k]] : 0x7FC0;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float x = __fsub_rn(__fmul_rn(bf2f(c4[k]), inv_t), M);
+                if (i4[k] < V && x >= floor_x) best_of(best, bi, gumbel_score(x, key, (uint32_t)i4[k]), (uint32_t)i4[k]);
+            }
+        }
+        block_best(best, bi, bv, bix);
+        if (t == 0) write_token(bi, token, greedy, pos, prompt);
+        return;
     }
     // threshold 0: every token is in the nucleus, and the draw is the best block winner
     if (t == 0) write_token(bix[0], token, greedy, pos, prompt);

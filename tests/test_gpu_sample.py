@@ -102,6 +102,9 @@ CASES = [  # (seed, V, kind, a, T, top_p)
     (22, 1000, "saturated", 1.0, 1.0, 0.9), (23, 65536, "mixed", 0.4, 1.0, 0.9), (24, 30000, "mixed", 0.45, 1.0, 0.6),
     (25, 65536, "mixed", 0.8, 1.0, 0.75), (26, 1500, "mixed", 0.9, 1.0, 0.4), (27, 1500, "mixed", 0.3, 0.9, 0.8),
     (28, 65536, "normal", 2e-4, 1.0, 0.9), (29, 1000, "two", 0.6, 0.05, 0.9), (30, 65536, "mixed", 0.1, 1.0, 0.95),
+    # the mass reached above 2^-10, and below -2^-10, in rows mostly between them; no cut
+    (31, 65536, "mixed", 0.7, 1.0, 0.15), (32, 1500, "mixed", 0.7, 1.0, 0.15), (33, 65536, "mixed", 0.7, 1.0, 0.98),
+    (34, 1500, "normal", 1.0, 1.0, 1.0),
 ]
 
 
