@@ -22,9 +22,10 @@
 //    the tiles.
 // It replaces one 128 x 64 tile with the dequantised W in LDS, whose workgroups moved 281 bytes of
 // LDS a cycle's worth of products (128 is the rate) and left most of the chip idle below 1000
-// tokens. Measured, q/k/v (3072 rows) / o (2048 rows) at K = 2048: 16 tokens 17.3 / 18.3 -> 5.1 /
-// 5.0 us, 100 tokens 18.0 / 19.0 -> 9.5 / 9.6, 400 tokens 18.9 / 19.9 -> 18.3 / 14.8, 2048 tokens
-// 45.0 / 33.0 -> 38.1 / 29.1; K = 4096, 2048 rows, 2048 tokens 65.9 -> 43.6. At 2048 tokens the
+// tokens. Measured (back to back in a graph), q/k/v (3072 rows, bf16 out) / o (2048 rows, += fp32) at
+// K = 2048: 16 tokens 17.9 / 19.2 -> 5.9 / 5.7 us, 100 tokens 18.5 / 19.7 -> 9.9 / 9.6, 400 tokens
+// 19.2 / 20.1 -> 18.3 / 13.7, 2048 tokens 44.2 / 33.3 -> 38.7 / 29.1; K = 4096, 2048 rows, 2048 tokens
+// 56.0 -> 43.1 (bf16 out). At 2048 tokens the
 // matrix cores are busy 27% of the time and LDS 38%: the dequantisation's VALU work adds to the
 // products (both waves of a SIMD are in the same part), and a workgroup starts and ends in 5 us.
 #include <type_traits>
@@ -304,18 +305,24 @@ int launch_gemm_q4_tile(const GemmArgs& a, int epi, hipStream_t st) {
 
 // The tile is the one of least modelled time: first + round * ceil(workgroups / 256), in tenths of a
 // us at K = 2048 (other K scale all alike), fitted to a sweep of 6 .. 2048 tokens at 2048 and 3072
-// rows, K = 2048 and 4096 (two of the smallest fit a CU, so that its rounds overlap). The tile chosen
-// was the fastest of the sweep, or within 5% of it. The last two take what the others' equal shares
-// and 32-bit offsets do not: the general instance of this kernel (3072 rows, K = 2112, 40 tokens: 10.9
-// us) and the kernel with the weights in LDS (17.8), which is faster from two rounds of the first on
-// (600 tokens 20.2 against 33.1).
-struct GemmTile { int m, n, ks, first, round; int (*launch)(const GemmArgs&, int, hipStream_t); };
+// rows, K = 2048 and 4096 (two of the smallest fit a CU, so that its rounds overlap). It leaves out how
+// full the last round is, up to a fifth of a round of the large tiles (256 workgroups of 128 x 192:
+// 37.8 us, 131 of them 31): over 1 .. 2048 tokens, 520 .. 3072 rows and K = 1024 .. 4096 the tile chosen
+// takes 0.1% more than the fastest of them on average, 6% at most. The last two take what the others'
+// equal shares and 32-bit offsets do not: the general instance of this kernel (3072 rows, K = 2112, 40
+// tokens: 11.0 us) and the kernel with the weights in LDS (18.4), which is faster from two rounds of the
+// first on (600 tokens 20.2 against 33.1).
+// Below K = 1024 the starts and ends that the model scales with K decide: the kernel with the weights in
+// LDS, which has the shortest, takes all but one round of the smaller tiles, from K = short_k (3072 rows,
+// K = 512, 600 tokens: 128 x 64 in registers 9.7 us, in LDS 8.5; K = 192, 16 tokens: the general instance
+// 6.0, in LDS 5.2; K = 512, 16 tokens: 64 x 32 6.4, in LDS 7.4): within 0.2% of the fastest on average.
+struct GemmTile { int m, n, ks, first, round, short_k; int (*launch)(const GemmArgs&, int, hipStream_t); };
 static const GemmTile GEMM_TILES[] = {
-    {16, 16, 8, 25, 25, launch_gemm_q4_tile<1, 1, 8>},    {32, 16, 8, 0, 58, launch_gemm_q4_tile<2, 1, 8>},
-    {64, 32, 4, 0, 83, launch_gemm_q4_tile<4, 1, 4>},    {64, 64, 4, 0, 114, launch_gemm_q4_tile<4, 2, 4>},
-    {128, 64, 2, 0, 158, launch_gemm_q4_tile<8, 1, 2>},  {128, 128, 2, 0, 205, launch_gemm_q4_tile<8, 2, 2>},
-    {128, 192, 2, 0, 304, launch_gemm_q4_tile<8, 3, 2>},
-    {64, 32, 0, 0, 100, launch_gemm_q4_tile<4, 1, 4, true>}, {128, 64, 0, 50, 130, launch_gemm_q4_lds},
+    {16, 16, 8, 25, 25, 1024, launch_gemm_q4_tile<1, 1, 8>},    {32, 16, 8, 0, 58, 1024, launch_gemm_q4_tile<2, 1, 8>},
+    {64, 32, 4, 0, 83, 512, launch_gemm_q4_tile<4, 1, 4>},    {64, 64, 4, 0, 114, 1024, launch_gemm_q4_tile<4, 2, 4>},
+    {128, 64, 2, 0, 158, 1024, launch_gemm_q4_tile<8, 1, 2>},  {128, 128, 2, 0, 205, 1024, launch_gemm_q4_tile<8, 2, 2>},
+    {128, 192, 2, 0, 304, 1024, launch_gemm_q4_tile<8, 3, 2>},
+    {64, 32, 0, 0, 100, 320, launch_gemm_q4_tile<4, 1, 4, true>}, {128, 64, 0, 50, 130, 0, launch_gemm_q4_lds},
 };
 
 int launch_gemm_q4(const GemmArgs& a, int epi, hipStream_t st) {
@@ -325,6 +332,7 @@ int launch_gemm_q4(const GemmArgs& a, int epi, hipStream_t st) {
     for (const GemmTile& t : GEMM_TILES) {
         if (t.ks && (!narrow || a.K / 64 % (2 * t.ks))) continue;
         const long long tiles = (((long long)a.T + t.m - 1) / t.m) * (((long long)a.O + t.n - 1) / t.n);
+        if (a.K < t.short_k || (a.K < 1024 && t.short_k && tiles > 256)) continue;
         const long long cost = t.first + (tiles + 255) / 256 * t.round;
         if (tiles <= 0x7FFFFFFFLL && (!best || cost < least)) best = &t, least = cost;
     }

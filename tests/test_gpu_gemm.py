@@ -112,8 +112,13 @@ def test_gemm_c5_qkv_sampled(torch_gpu, orc):
 @pytest.mark.parametrize("T,O,K,shift", [
     (5, 33, 1024, 0), (5, 33, 4096, 0), (64, 2048, 1024, 0),      # 16 x 16 (one and two panels of scales), 32 x 16
     (130, 1000, 512, 0), (300, 2050, 4096, 0),                    # 64 x 32, 64 x 64 with a second panel
-    (300, 2050, 256, 2), (1030, 2000, 256, 0), (1300, 3000, 256, 0),   # 128 x 64, x 128, x 192
-    (1, 5, 64, 2), (70, 100, 192, 2), (1100, 2100, 320, 0),       # the general instance, uneven shares; W in LDS
+    (300, 2050, 256, 2), (1030, 2000, 256, 0), (1300, 3000, 256, 0),   # few inputs: W in LDS
+    (1, 5, 64, 2), (70, 100, 192, 2), (1100, 2100, 320, 0),
+    (600, 2050, 1024, 2), (1030, 2000, 1280, 0), (1300, 3000, 1024, 0),   # 128 x 64, x 128, x 192
+    (5, 33, 6144, 0), (130, 1000, 6144, 2), (600, 2050, 6144, 0),   # a third panel, in the first one's place
+    (1, 5, 320, 2), (70, 100, 576, 2),                            # the general instance: shares of 2, 2, 1, 0 and 4, 4, 1, 0 groups
+    (33, 70, 3840, 0), (33, 70, 6208, 2), (33, 70, 6208, 0),      # several panels, the first case's by whole words
+    (300, 520, 256, 0), (300, 520, 512, 0), (300, 520, 960, 0), (300, 520, 1088, 0),   # either side of K = 320, 512 and 1024
 ])
 def test_gemm_tiles(torch_gpu, orc, T, O, K, shift):
     """Every tile the rule can choose, at ragged sizes: rows and tokens past the last tile's edge,
@@ -136,3 +141,21 @@ def test_gemm_tiles(torch_gpu, orc, T, O, K, shift):
         got = Y.float().cpu().numpy()
         check(got[:, :O], orc, w, s, b, X, rows, epi)
         assert (got[:, O:] == 7.0).all()
+
+
+def test_gemm_rows_past_32_bit_offsets(torch_gpu, orc):
+    """X rows so far apart that a tile's reach past 4 GB: the general instance's 64-bit offsets, over a
+    multiple of the inputs that the tiles with 32-bit ones would take."""
+    from embla_attn import ops
+    torch = torch_gpu
+    T, O, K, ldx = 66, 40, 2048, (1 << 25) + 8
+    g = synth.SplitMix64(53)
+    w, s, b = synth.q4_weights(g, O, K)
+    X = synth.bf16_bits(g.normal(T * K).astype(np.float32)).reshape(T, K)
+    buf, offs = pack(w, s, b)
+    Xs = torch.empty((T - 1) * ldx + K, dtype=torch.bfloat16, device="cuda")
+    Xs.as_strided((T, K), (ldx, 1)).copy_(dev(X, torch.bfloat16).reshape(T, K))
+    Y = torch.empty((T, O), dtype=torch.float32, device="cuda")
+    say("gemm rows past 32-bit offsets")
+    ops.gemm_q4(dev(buf), offs, Xs, Y, T, O, K, 4, ldx=ldx)
+    check(Y.cpu().numpy(), orc, w, s, b, X, [0, 31, 32, 63, 64, 65], 4)
