@@ -164,13 +164,19 @@ def test_q_prep_b_head_major(torch_gpu, orc):
             np.testing.assert_array_equal(got[h, t], want, err_msg=f"t={t} h={h}")
 
 
+# chunks of up to 512 tokens take the unstaged kernel with either workspace; of the longer ones 513 and
+# 577 tokens split in 7 and 6 (the merge of a row a wave), the ends fill a tile of 128 or leave 1 to 127
 @pytest.mark.parametrize("p0,T,tight", [(0, 100, False), (1000, 96, False), (2100, 64, False), (2500, 1, False),
-                                         (100, 100, True), (30720, 2048, False)])
+                                         (100, 100, True), (30720, 2048, False),
+                                         (0, 512, True), (0, 513, False), (37, 513, True), (2500, 513, True),
+                                         (2500, 577, False), (1000, 520, True), (1000, 700, False), (37, 700, True),
+                                         (512, 512, False), (511, 513, False), (0, 2100, True)])
 def test_prefill_staged_copy_bit_identical(torch_gpu, orc, p0, T, tight):
     """With a workspace that holds the staged fp16 copy, the region is converted once
     (prestage_kernel) and attended through the 16-bit tile path: the products are the ones each
     workgroup's own staging forms, so the output is bit for bit the unstaged path's; positions
-    past p0 + T (never written: NaN scales) stay out of it."""
+    past p0 + T (never written: NaN scales) stay out of it. The copy is made for chunks of more than
+    512 tokens."""
     from embla_attn import ops
     torch = torch_gpu
     say(f"prefill staged copy p0={p0} T={T} tight={tight}")
@@ -190,7 +196,15 @@ def test_prefill_staged_copy_bit_identical(torch_gpu, orc, p0, T, tight):
     staged = ops.prefill_int8(q, kc, vc, T, p0, max_s, 4, ws=wss)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(staged.view(torch.int16).cpu().numpy(), plain.view(torch.int16).cpu().numpy())
+    copy = wss.buf[(ops.PrefillWorkspace(T, 16).nbytes + 255) // 256 * 256:]
+    assert bool((copy != 0xFF).any()) == (T > 512)
+    K, ks, V, vs = cache_after_chunk(orc, c)
     if T <= 100:
-        K, ks, V, vs = cache_after_chunk(orc, c)
         ref = orc.prefill_int8(synth.bf16_val(c["q"]), K, ks, V, vs, p0, weights=0)
         assert_close(bf16_host(staged), ref, what=f"staged p0={p0} T={T}")
+    elif p0 < 30720:
+        got = bf16_host(staged)
+        for i in chunk_rows(T):
+            pos = p0 + i
+            ref = orc.decode_int8(synth.bf16_val(c["q"][i]), K[:, :pos + 1], ks[:, :pos + 1], V[:, :pos + 1], vs[:, :pos + 1])
+            assert_close(got[i], ref, what=f"staged p0={p0} T={T} row {i}")

@@ -1,7 +1,8 @@
 """Seeded random shapes against the oracle: decode over int8 caches at random lengths, capacities
-and chunkings; prefill at random prefix lengths and chunk sizes, staged and unstaged (bit-equal to
-each other); the sparse-layer decode at random lengths, its selection bit for bit. The cases are
-drawn once from fixed seeds, so a failure names a reproducible shape."""
+and chunkings; prefill at random prefix lengths and chunk sizes, with room for the staged copy (made
+from 513 tokens on) and without (bit-equal to each other); the sparse-layer decode at random lengths,
+its selection bit for bit. The cases are drawn once from fixed seeds, so a failure names a
+reproducible shape."""
 import random
 
 import numpy as np
@@ -33,6 +34,9 @@ def _prefill_cases():
     for i in range(5):
         p0, T = rng.randint(0, 5000), rng.randint(1, 300)
         out.append((400 + i, p0, T, (p0 + T + 31) // 32 * 32 + 32 * rng.randint(0, 2)))
+    for i in range(3):   # chunks that are staged
+        p0, T = rng.randint(0, 2000), rng.randint(513, 800)
+        out.append((410 + i, p0, T, (p0 + T + 31) // 32 * 32 + 32 * rng.randint(0, 2)))
     return out
 
 
