@@ -678,9 +678,10 @@ int embla_prefill_int8(const void* q, int q_dtype, long q_tok_stride, long q_hea
     a.q_bf16 = q_dtype == EMBLA_BF16; a.out_bf16 = o_dtype == EMBLA_BF16;
     // a workspace large enough for the staged copy: the region's keys are converted to fp16 once
     // (prestage_kernel) instead of once a workgroup, for the instances that have a staged form and
-    // chunks with enough workgroups a key to pay for the pass (40 tokens after 30000 keys: 50.8 us
-    // staged, 33.6 not; 193 after 7003 39.8, 35.7; 400 after 1000 34.0, 31.4; 700 after 10000 96.7,
-    // 97.8; 1200 after 20000 232, 237); the products are the same
+    // chunks with enough workgroups a key to pay for the pass (40 tokens after 30000 keys: 48.0 us
+    // staged, 34.0 not; 193 after 7003 40.0, 38.4; 400 after 1000 36.0, 32.7; 512 after 30000 148, 142;
+    // 700 after 10000 84.7, 84.6, after 30000 200, 202; 1200 after 20000 228, 234; 1400 278, 313); the
+    // products are the same
     const size_t staged = embla_prefill_staged_workspace_bytes(T, p0, n_q, n_kv);
     if (ws && staged && ws_bytes >= staged && window == 0 && !a.relu2 && !a.scale32 && a.q_bf16 && a.out_bf16 &&
         n_q == 4 * n_kv && T > kStageMinTokens) {

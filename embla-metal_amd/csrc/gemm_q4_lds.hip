@@ -1,5 +1,6 @@
-// The 4-bit projections at prefill for a number of input groups that the tiles of gemm_q4.hip do
-// not divide, or rows too long for their offsets: the same product (gemm.metal:1-134), any K.
+// The 4-bit projections at prefill for few inputs (under 1024), a number of input groups that the tiles
+// of gemm_q4.hip do not divide, or rows too long for their offsets: the same product
+// (gemm.metal:1-134), any K.
 //
 // MI355X design. A workgroup computes 128 tokens x 64 rows with 4 waves, each a 64 x 32 block as
 // 2 tiles of v_mfma_f32_32x32x16_bf16 (A: X rows, B: W rows, so both operands are 16-byte row
@@ -18,24 +19,22 @@ namespace embla {
 typedef __bf16 bf8v_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
 
-constexpr int QM = 128, QK = 64;             // tokens, inputs a step (rows: the template's QN)
+constexpr int QM = 128, QN = 64, QK = 64;    // tokens, rows, inputs a step
 constexpr int QROW = QK + 8;                 // bf16 elements an LDS row (144 bytes)
 
-template <int QN>
 struct GemmLdsSmem {
     uint16_t x[2][QM * QROW];
     uint16_t w[2][QN * QROW];
 };
 
-template <int EPI, int QN>
+template <int EPI>
 __global__ __launch_bounds__(256, 2) void gemm_q4_lds_kernel(GemmArgs a) {
-    constexpr int J = QN / 64;            // 32-row tiles a wave
-    constexpr int WPT = QN / 32;          // W words a staging thread: 4 or 2
+    constexpr int WPT = 2;                // W words a staging thread
     constexpr int TPR = 8 / WPT;          // staging threads a W row
-    __shared__ __attribute__((aligned(16))) GemmLdsSmem<QN> sm;
+    __shared__ __attribute__((aligned(16))) GemmLdsSmem sm;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int n0 = blockIdx.x * QN, m0 = blockIdx.y * QM;
-    const int wm = (wv >> 1) * 64, wn = (wv & 1) * (QN / 2);   // the wave's 64 x QN/2 block
+    const int wm = (wv >> 1) * 64, wn = (wv & 1) * (QN / 2);   // the wave's 64 x 32 block
     // X staging: chunk 256 i + tid is row 32 i + tid / 8, columns 8 (tid % 8) .. +7, so one
     // wave load reads 8 whole 128-byte row pieces
     const int sr = tid >> 3, sc = 8 * (tid & 7);
@@ -55,15 +54,9 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_lds_kernel(GemmArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; i++) R.x[i] = ld16(xr[i] + k0);
         const uint32_t* wp = (const uint32_t*)(W + a.wo) + wrow * wpr + k0 / 8 + WPT * (tid % TPR);
-        if constexpr (WPT == 4) {
-            const u4_t v = ld16(wp);
-#pragma unroll
-            for (int j = 0; j < 4; j++) R.w[j] = v[j];
-        } else {
-            const u2_t v = ld8(wp);
-            R.w[0] = v[0];
-            R.w[1] = v[1];
-        }
+        const u2_t v = ld8(wp);
+        R.w[0] = v[0];
+        R.w[1] = v[1];
         R.s = bf2f(*(const uint16_t*)(W + a.so + (wrow * gpr + k0 / 64) * 2));
         R.b = bf2f(*(const uint16_t*)(W + a.bo + (wrow * gpr + k0 / 64) * 2));
     };
@@ -85,30 +78,22 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_lds_kernel(GemmArgs a) {
         }
     };
 
-    f16_t acc[2][J];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < J; j++) acc[i][j] = (f16_t){};
+    f16_t acc[2] = {};
     const int fr = lane & 31, fk = 8 * (lane >> 5);   // operand row within a tile, k offset
     auto compute = [&](int buf) {   // every operand of the step read first, then the products
-        bf8v_t fa[QK / 16][2], fb[QK / 16][J];
+        bf8v_t fa[QK / 16][2], fb[QK / 16];
 #pragma unroll
         for (int kk = 0; kk < QK / 16; kk++) {
 #pragma unroll
             for (int i = 0; i < 2; i++)
                 fa[kk][i] = *(const bf8v_t*)(sm.x[buf] + (wm + 32 * i + fr) * QROW + 16 * kk + fk);
-#pragma unroll
-            for (int j = 0; j < J; j++)
-                fb[kk][j] = *(const bf8v_t*)(sm.w[buf] + (wn + 32 * j + fr) * QROW + 16 * kk + fk);
+            fb[kk] = *(const bf8v_t*)(sm.w[buf] + (wn + fr) * QROW + 16 * kk + fk);
         }
 #pragma unroll
         for (int kk = 0; kk < QK / 16; kk++)
 #pragma unroll
             for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < J; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk][i], fb[kk][j], acc[i][j], 0, 0, 0);
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk][i], fb[kk], acc[i], 0, 0, 0);
     };
     const int steps = a.K / QK;
     // step st computes buffer st & 1 and stores step st + 1 (loaded at st - 1) into the other;
@@ -118,18 +103,15 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_lds_kernel(GemmArgs a) {
     const int last = QK * (steps - 1);
     // EPI 2 (+=): the residual's items are requested first, so that their reads overlap the
     // products instead of following them
-    float yp[EPI == 2 ? 2 : 1][EPI == 2 ? J : 1][16];
+    const int n = n0 + wn + fr;   // the lane's row of W
+    float yp[EPI == 2 ? 2 : 1][16];
     if constexpr (EPI == 2) {
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int j = 0; j < J; j++) {
-                const int n = min(n0 + wn + 32 * j + fr, a.O - 1);
-#pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    const int m = min(m0 + wm + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3), a.T - 1);
-                    yp[i][j][e] = ((const float*)a.Y)[(size_t)m * a.ldy + n];
-                }
+            for (int e = 0; e < 16; e++) {
+                const int m = min(m0 + wm + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3), a.T - 1);
+                yp[i][e] = ((const float*)a.Y)[(size_t)m * a.ldy + min(n, a.O - 1)];
             }
     }
     load(0, R0);
@@ -148,40 +130,35 @@ __global__ __launch_bounds__(256, 2) void gemm_q4_lds_kernel(GemmArgs a) {
         __syncthreads();
     }
 
-    // epilogue: tile (i, j) item e of lane l is token wm + 32 i + 8 (e / 4) + 4 (l / 32) + e % 4,
-    // row wn + 32 j + l % 32
+    // epilogue: tile i item e of lane l is token wm + 32 i + 8 (e / 4) + 4 (l / 32) + e % 4, row
+    // wn + l % 32
+    if (n >= a.O) return;
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < J; j++) {
-            const int n = n0 + wn + 32 * j + fr;
-            if (n >= a.O) continue;
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const int m = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-                if (m >= a.T) continue;
-                const float v = acc[i][j][e];
-                const size_t at = (size_t)m * a.ldy + n;
-                if constexpr (EPI == 0) ((uint16_t*)a.Y)[at] = f2bf(v);
-                else if constexpr (EPI == 1) {
-                    const float t = fmaxf(bf2f(f2bf(v)), 0.0f);
-                    ((uint16_t*)a.Y)[at] = f2bf(t * t);
-                } else if constexpr (EPI == 2) ((float*)a.Y)[at] = yp[i][j][e] + bf2f(f2bf(v));
-                else if constexpr (EPI == 3) ((float*)a.Y)[at] = bf2f(f2bf(v));
-                else ((float*)a.Y)[at] = v;
-            }
+        for (int e = 0; e < 16; e++) {
+            const int m = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+            if (m >= a.T) continue;
+            const float v = acc[i][e];
+            const size_t at = (size_t)m * a.ldy + n;
+            if constexpr (EPI == 0) ((uint16_t*)a.Y)[at] = f2bf(v);
+            else if constexpr (EPI == 1) {
+                const float t = fmaxf(bf2f(f2bf(v)), 0.0f);
+                ((uint16_t*)a.Y)[at] = f2bf(t * t);
+            } else if constexpr (EPI == 2) ((float*)a.Y)[at] = yp[i][e] + bf2f(f2bf(v));
+            else if constexpr (EPI == 3) ((float*)a.Y)[at] = bf2f(f2bf(v));
+            else ((float*)a.Y)[at] = v;
         }
 }
 
 int launch_gemm_q4_lds(const GemmArgs& a, int epi, hipStream_t st) {
-    constexpr int QN = 64;
     const dim3 grid((a.O + QN - 1) / QN, (a.T + QM - 1) / QM), block(256);
     switch (epi) {
-        case 0: hipLaunchKernelGGL((gemm_q4_lds_kernel<0, QN>), grid, block, 0, st, a); break;
-        case 1: hipLaunchKernelGGL((gemm_q4_lds_kernel<1, QN>), grid, block, 0, st, a); break;
-        case 2: hipLaunchKernelGGL((gemm_q4_lds_kernel<2, QN>), grid, block, 0, st, a); break;
-        case 3: hipLaunchKernelGGL((gemm_q4_lds_kernel<3, QN>), grid, block, 0, st, a); break;
-        case 4: hipLaunchKernelGGL((gemm_q4_lds_kernel<4, QN>), grid, block, 0, st, a); break;
+        case 0: hipLaunchKernelGGL((gemm_q4_lds_kernel<0>), grid, block, 0, st, a); break;
+        case 1: hipLaunchKernelGGL((gemm_q4_lds_kernel<1>), grid, block, 0, st, a); break;
+        case 2: hipLaunchKernelGGL((gemm_q4_lds_kernel<2>), grid, block, 0, st, a); break;
+        case 3: hipLaunchKernelGGL((gemm_q4_lds_kernel<3>), grid, block, 0, st, a); break;
+        case 4: hipLaunchKernelGGL((gemm_q4_lds_kernel<4>), grid, block, 0, st, a); break;
         default: return EMBLA_ERR_INVALID;
     }
     return hipGetLastError() == hipSuccess ? EMBLA_OK : EMBLA_ERR_HIP;

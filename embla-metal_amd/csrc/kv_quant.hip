@@ -36,14 +36,15 @@ __global__ __launch_bounds__(64) void kv_quant_kernel(KVQuantArgs a) {
     store_pair8(rows, a.n_kv, a.max_s, h, pos, is_v, a.row_major, a.scale32, q0, q1, am, lane);
 }
 
-// waves a tile and rows a wave: a wave's rows are one serial chain (2048 tokens of 4 heads: 6.2 us at 4
-// waves, 5.6 at 8, 5.2 at 16)
+// waves a tile and rows a wave: a wave's rows are one serial chain (int8, 1024 / 2048 tokens of 4 heads:
+// 5.3 / 6.4 us at 4 waves, 4.6 / 5.8 at 8, 4.35 / 5.7 at 16; ring with the pre-ops 4.6 / 5.7, 4.15 / 5.5,
+// 4.1 / 5.55)
 constexpr int TW = 16, TR = 32 / TW;
 
 /// The same rows a 32-position tile at a time: a workgroup a (tile, kv head, K or V) quantises its
 /// rows into LDS and writes the tile in whole 16-byte pieces. A wave a row stores V's bytes one by
-/// one, 128 cache lines a row, and a 2048-token chunk of 4 heads is 16384 workgroups: 8.2 us where
-/// this takes 5.2. A chunk's first and last tile may be partial: K's (and a row-major cache's) pieces
+/// one, 128 cache lines a row, and a 2048-token chunk of 4 heads is 16384 workgroups: 7.15 us where
+/// this takes 5.7. A chunk's first and last tile may be partial: K's (and a row-major cache's) pieces
 /// belong to one position each, V's are then stored byte by byte.
 template <bool ROW_MAJOR>
 __global__ __launch_bounds__(64 * TW) void kv_quant_tile_kernel(KVQuantArgs a) {
@@ -109,10 +110,12 @@ __global__ __launch_bounds__(64 * TW) void kv_quant_tile_kernel(KVQuantArgs a) {
     }
 }
 
-/// Rows (tokens x heads) above which an append goes a 32-position tile at a time; below, the tile's
-/// barrier and its second pass cost more than whole pieces save (us, a wave a row / a tile): int8, 4
-/// heads, 512 tokens 3.6 / 3.9, 1024 5.0 / 4.8, 2048 7.4 / 6.2; 2 heads, 2048 5.0 / 5.2; ring with
-/// the pre-ops, 4 heads, 512 3.8 / 4.0, 1024 5.2 / 4.3, 2048 7.3 / 5.8.
+/// Rows (tokens x heads) above which an append goes a 32-position tile at a time; for few, the tile's
+/// barrier and its second pass cost more than whole pieces save (us, a wave a row / a tile, at 1 to 8
+/// heads alike): int8, 2048 rows 3.7 / 4.1, 3072 4.3 / 4.2, 4096 4.95 / 4.4 (fp32 scales 4.9 / 4.7), 8192
+/// 7.15 / 5.7; ring 1024 2.8 / 3.2, 1536 3.1 / 3.2, 2048 3.4 / 3.2, 8192 5.9 / 4.25; ring with the
+/// pre-ops 1024 3.5 / 3.8, 1536 4.1 / 3.9, 2048 4.4 / 3.9, 8192 8.7 / 5.55. Both lines lie a little above
+/// where the two are equal (3000 and 1500), so that every call from there on gains.
 constexpr int KV_TILE_ROWS = 4096, RING_TILE_ROWS = 2048;
 
 int launch_kv_quant(const KVQuantArgs& a, hipStream_t st) {
@@ -188,7 +191,7 @@ __global__ __launch_bounds__(64) void ring_append_kernel(RingAppendArgs a) {
 
 /// The same rows a 32-slot tile at a time (kv_quant_tile_kernel's way): a workgroup a (tile, head, K
 /// or V), its rows into LDS, then whole 16-byte pieces; the tile's RoPE angles are evaluated once, into
-/// LDS. 2048 rows of 4 heads with the pre-ops: 7.9 us a wave a row, 5.2 this way.
+/// LDS. 2048 tokens of 4 heads with the pre-ops: 8.7 us a wave a row, 5.55 this way.
 __global__ __launch_bounds__(64 * TW) void ring_append_tile_kernel(RingAppendArgs a) {
     constexpr int RS = HD + 8;   // elements a row in LDS: 16-byte reads of 16 rows on distinct banks
     __shared__ __attribute__((aligned(16))) uint16_t rows[32 * RS];

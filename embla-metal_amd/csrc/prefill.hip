@@ -114,6 +114,7 @@ template <int GQ, bool RELU2, bool SCALE32, bool QBF, bool OBF, bool RING = fals
 __global__ __launch_bounds__(64 * PF_WAVES, 1) void prefill_int8_kernel(PrefillArgs a) {
     constexpr int NT = 64 * PF_WAVES;
     constexpr int RB = PF_WAVES / GQ;                       // 32-row blocks a workgroup
+    static_assert(RING || !RELU2, "an int8 region's ReLU² prefill: relu2_prefill_kernel");
     __shared__ PrefillSmem sm;
     // full caches: consecutive workgroup ids go to consecutive XCDs, and id % (n_kv * nsplit)
     // picks the (kv head, split), so that each XCD streams as few key ranges as possible and its L2
@@ -351,7 +352,7 @@ __global__ __launch_bounds__(64 * PF_WAVES, 1) void prefill_int8_kernel(PrefillA
     // exactly representable in fp16 (any shift of a row's scores leaves its softmax unchanged).
     // Its range is fp16's: scores up to 65504 in log2 units (about 45,400 before the 1/sqrt(d)
     // scale); the layers' q and k are RMS-normed a head, which keeps scores far below that.
-    constexpr bool FOLD = PF_FOLD && !RELU2 && !BF && (!RING || LIN);
+    constexpr bool FOLD = PF_FOLD && !BF && (!RING || LIN);
     const u4_t kone = {h ? 0u : 0x3C00u, 0u, 0u, 0u};   // fp16 1.0 at k 0
     u4_t qm = {0u, 0u, 0u, 0u};                          // -m (0 while the row has no key)
     f16_t O[4];
@@ -434,8 +435,8 @@ __global__ __launch_bounds__(64 * PF_WAVES, 1) void prefill_int8_kernel(PrefillA
             // a ring's scores are unscaled (x c): ReLU² scales them here, softmax in the exponent
 #pragma unroll
             for (int e = 0; e < 16; e++) {
-                x[e] = RING && RELU2 ? s0[e] * cr : s0[e];
-                x[16 + e] = RING && RELU2 ? s1[e] * cr : s1[e];
+                x[e] = RELU2 ? s0[e] * cr : s0[e];
+                x[16 + e] = RELU2 ? s1[e] * cr : s1[e];
             }
             if (!full_tile) {   // uniform: only the diagonal (and window-edge) tiles
 #pragma unroll

@@ -5,9 +5,9 @@
 // MI355X design: a workgroup is 32 RB query rows (4 RB tokens x the kv head's 8 query heads) and its 8
 // waves deal the 32-key blocks among themselves, each wave with its own O for all the rows: ReLU²
 // weights need no running maximum, so the waves' sums add up at the end (through LDS) and the key
-// loop has no barrier and no LDS tile. The entry point takes no workspace, so keys cannot be split
-// over workgroups: splitting them over a workgroup's waves keeps every SIMD busy from few tokens on,
-// where a workgroup of 32 tokens with all its waves on the same LDS tile left half the chip idle at
+// loop has no barrier and no LDS tile. Keys are not split over workgroups (the reference's entry point
+// takes no workspace; where one is given it is not used): splitting them over a workgroup's waves keeps
+// every SIMD busy from few tokens on, where a workgroup of 32 tokens with all its waves on the same LDS tile left half the chip idle at
 // 2048 tokens, and took a short chunk through the whole key range at one workgroup's pace.
 // S^T = K·Q^T and O^T += V^T·P^T run on v_mfma_f32_32x32x16_f16 with query rows as columns; a
 // wave's 16-byte loads of the int8 tiles are its operands: the k-slots of each product follow the

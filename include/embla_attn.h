@@ -194,10 +194,11 @@ int embla_sparse_layer_decode(const void* q, const void* qi, const float* w, con
  * Query row (t, h) at q + t * q_tok_stride + h * q_head_stride (elements, q_dtype), output row at
  * o + t * o_tok_stride + h * o_head_stride (o_dtype). weights: EMBLA_SOFTMAX, or EMBLA_RELU2_SINK
  * (threshold 0, sink sqrt(128), as relu2_prefill_nax, attn_nax.metal:61-364). n_q / n_kv in {4, 8}.
- * ws (optional, embla_prefill_workspace_bytes(T, n_q)): lets the key range split (partial rows
- * merged by a second launch) until every CU has a workgroup, 64 splits at most; NULL: one pass. A
- * workspace of at least 4 T n_q 132 floats but less than that many bytes: the splits it has room
- * for. */
+ * ws (optional, embla_prefill_workspace_bytes(T, n_q)): lets the key range split where its
+ * workgroups leave CUs idle, into up to 64 parts whose partial rows a second launch merges (in
+ * fp32; two parts of a range of 512 keys or more as fp16 O / l); NULL: one pass. A workspace of at
+ * least 4 T n_q 132 floats but less than that many bytes: the splits it has room for. Not used with
+ * EMBLA_RELU2_SINK. */
 int embla_prefill_int8(const void* q, int q_dtype, long q_tok_stride, long q_head_stride, const void* kc,
                        const void* vc, void* o, int o_dtype, long o_tok_stride, long o_head_stride, int T, int p0,
                        int max_s, int n_q, int n_kv, int weights, int scale_dtype, int window, void* ws,
@@ -210,7 +211,8 @@ size_t embla_prefill_workspace_bytes(int T, int n_q);
  * counterpart in the reference, whose threadgroups each widen the int8 rows they stage,
  * attn_nax.metal:26-56): embla_prefill_int8 / embla_prefill_full given at least this much convert
  * the region once into it, bit-identical products, and attend over the copy (softmax, fp16
- * scales, bf16 q and out, n_q = 4 n_kv, no window; other calls ignore the extra bytes). */
+ * scales, bf16 q and out, n_q = 4 n_kv, no window, more than 512 tokens; other calls ignore the
+ * extra bytes). */
 size_t embla_prefill_staged_workspace_bytes(int T, int p0, int n_q, int n_kv);
 
 /* Full-layer prefill chunk (config C5 full): the chunk's bf16 K and V [T][n_kv][128] quantised into
