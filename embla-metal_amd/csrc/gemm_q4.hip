@@ -26,7 +26,7 @@
 // K = 2048: 16 tokens 17.9 / 19.2 -> 5.9 / 5.7 us, 100 tokens 18.5 / 19.7 -> 9.9 / 9.6, 400 tokens
 // 19.2 / 20.1 -> 18.3 / 13.7, 2048 tokens 44.2 / 33.3 -> 38.7 / 29.1; K = 4096, 2048 rows, 2048 tokens
 // 56.0 -> 43.1 (bf16 out). At 2048 tokens the
-// matrix cores are busy 27% of the time and LDS 38%: the dequantisation's VALU work adds to the
+// matrix cores are busy 29% of the time and LDS about 40%: the dequantisation's VALU work adds to the
 // products (both waves of a SIMD are in the same part), and a workgroup starts and ends in 5 us.
 #include <type_traits>
 #include "common.hpp"
